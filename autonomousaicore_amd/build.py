@@ -40,10 +40,11 @@ def _obj(src: str) -> str:
     return os.path.join(BUILD, rel + ".o")
 
 
-# Per-file code generation options.  attention.hip: MFMAs in the VGPR form, so that the
+# Per-file code generation options.  attention.hip, attention_general.hip: MFMAs in the VGPR form, so that the
 # backward's long-lived dK/dV accumulators are not copied between VGPRs and AGPRs around every
 # MFMA of the inner loop (the AGPR form's register assignment does that for these kernels).
-FILE_FLAGS = {"attention.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]}
+FILE_FLAGS = {"attention.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
+              "attention_general.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]}
 
 
 def _compile(src: str) -> tuple[str, int, str]:

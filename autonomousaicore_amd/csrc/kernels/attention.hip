@@ -24,7 +24,8 @@
 //              [query x key] so a lane owns a key and P / dS feed dV^T += dO^T P and
 //              dK^T += Q^T dS from registers.
 //              dQ:   one block = 128 queries over 64-key tiles (dQ^T += K^T dS^T).
-// fp32 path (the fp32 reference configuration, head_dim 16/32/64/128): SIMT kernels, fp32 math.
+// Everything else (fp32, head_dim 16 and 32, queries and keys of different lengths, the KV cache)
+// runs the kernels of attention_general.hip.
 #include <algorithm>
 #include <cmath>
 #include <type_traits>
@@ -410,60 +411,6 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_pipe(const bf16* __restrict__
 #pragma unroll
         for (int ob = 0; ob < OB; ++ob) store_t(op, oacc[ob], ob, inv);
         if (hl == 0) lse[(static_cast<int64_t>(b) * H + h) * S + myq] = (m_run * c + log2f(l_run)) * kLn2;
-    }
-}
-
-// D[b,h,s] = sum_d dO * O  (fp32), one wave per (token, head).
-template <typename T>
-__global__ __launch_bounds__(256) void attn_dot_k(const T* __restrict__ o, const T* __restrict__ dout, int64_t ldo,
-                                                  float* __restrict__ D, int64_t Ttok, int H, int S, int HD) {
-    const int64_t gw = (static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x) >> 6;
-    const int lane = threadIdx.x & 63;
-    if (gw >= Ttok * H) return;
-    const int64_t t = gw / H;
-    const int h = static_cast<int>(gw % H);
-    float acc = 0.0f;
-    for (int d = lane; d < HD; d += 64) {
-        const int64_t i = t * ldo + static_cast<int64_t>(h) * HD + d;
-        acc += ld(o, i) * ld(dout, i);
-    }
-    acc = wave_sum(acc);
-    if (lane == 0) {
-        const int64_t b = t / S, s = t % S;
-        D[(b * H + h) * S + s] = acc;
-    }
-}
-
-// The same for bf16 rows of HD % 8 == 0 elements with 16-byte loads: HD / 8 lanes per
-// (token, head) row, 64 / (HD / 8) rows per wave; each lane's eight products, then a
-// butterfly over the row's lanes.
-template <int HD>
-__global__ __launch_bounds__(256) void attn_dot_v8_k(const bf16* __restrict__ o, const bf16* __restrict__ dout,
-                                                     int64_t ldo, float* __restrict__ D, int64_t Ttok, int H, int S) {
-    constexpr int LPR = HD / 8, RPW = 64 / LPR;
-    const int64_t gw = (static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x) >> 6;
-    const int lane = threadIdx.x & 63, sub = lane % LPR;
-    const int64_t row = gw * RPW + lane / LPR;
-    const bool ok = row < Ttok * H;
-    float acc = 0.0f;
-    if (ok) {
-        const int64_t t = row / H;
-        const int h = static_cast<int>(row % H);
-        const int64_t i = t * ldo + static_cast<int64_t>(h) * HD + sub * 8;
-        const uint4 a = *reinterpret_cast<const uint4*>(o + i), b = *reinterpret_cast<const uint4*>(dout + i);
-        const uint32_t wa[4] = {a.x, a.y, a.z, a.w}, wb[4] = {b.x, b.y, b.z, b.w};
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            acc += __uint_as_float(wa[q] << 16) * __uint_as_float(wb[q] << 16);
-            acc += __uint_as_float(wa[q] & 0xffff0000u) * __uint_as_float(wb[q] & 0xffff0000u);
-        }
-    }
-#pragma unroll
-    for (int w = LPR / 2; w > 0; w >>= 1) acc += __shfl_xor(acc, w);
-    if (ok && sub == 0) {
-        const int64_t t = row / H, b = t / S, s = t % S;
-        const int h = static_cast<int>(row % H);
-        D[(b * H + h) * S + s] = acc;
     }
 }
 
@@ -900,294 +847,11 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dq_mfma(const bf16* __restric
     }
 }
 
-// ---------------------------------------------------------------------------------------
-// SIMT path (fp32 configuration, any dtype, head_dim 16/32/64/128): one thread per query row
-// (forward, dQ) or key row (dK, dV); fp32 math; K/V or Q/dO tiles staged in LDS.
-// ---------------------------------------------------------------------------------------
-constexpr int kSimtTile = 64;
-
-template <typename T, int HD>
-__global__ __launch_bounds__(64) void attn_fwd_simt(const T* __restrict__ q, const T* __restrict__ k,
-                                                    const T* __restrict__ v, int64_t ldq, int64_t ldk,
-                                                    T* __restrict__ o, int64_t ldo, float* __restrict__ lse, int H,
-                                                    int S, int Sk, float scale, int causal) {
-    __shared__ float sk[kSimtTile][HD + 1];
-    __shared__ float sv[kSimtTile][HD + 1];
-    const int h = blockIdx.y, b = blockIdx.z;
-    const int qi = blockIdx.x * kSimtTile + threadIdx.x;
-    const int64_t tok0 = static_cast<int64_t>(b) * S, tok0k = static_cast<int64_t>(b) * Sk;
-    const int64_t hoff = static_cast<int64_t>(h) * HD;
-    float qv[HD], acc[HD];
-    for (int d = 0; d < HD; ++d) {
-        qv[d] = qi < S ? ld(q, (tok0 + qi) * ldq + hoff + d) : 0.0f;
-        acc[d] = 0.0f;
-    }
-    float m = -INFINITY, l = 0.0f;
-    const int kend = causal ? min(Sk, static_cast<int>((blockIdx.x + 1) * kSimtTile)) : Sk;
-    for (int k0 = 0; k0 < kend; k0 += kSimtTile) {
-        __syncthreads();
-        for (int e = threadIdx.x; e < kSimtTile * HD; e += 64) {
-            const int r = e / HD, d = e % HD;
-            const int key = k0 + r;
-            sk[r][d] = key < Sk ? ld(k, (tok0k + key) * ldk + hoff + d) : 0.0f;
-            sv[r][d] = key < Sk ? ld(v, (tok0k + key) * ldk + hoff + d) : 0.0f;
-        }
-        __syncthreads();
-        if (qi >= S) continue;
-        for (int r = 0; r < kSimtTile; ++r) {
-            const int key = k0 + r;
-            if (key >= Sk || (causal && key > qi)) break;
-            float sdot = 0.0f;
-            for (int d = 0; d < HD; ++d) sdot += qv[d] * sk[r][d];
-            const float x = sdot * scale;
-            const float mn = fmaxf(m, x);
-            const float a = expf(m - mn);
-            const float p = expf(x - mn);
-            l = l * a + p;
-            for (int d = 0; d < HD; ++d) acc[d] = acc[d] * a + p * sv[r][d];
-            m = mn;
-        }
-    }
-    if (qi < S) {
-        for (int d = 0; d < HD; ++d) st(o, (tok0 + qi) * ldo + hoff + d, acc[d] / l);
-        lse[(static_cast<int64_t>(b) * H + h) * S + qi] = m + logf(l);
-    }
-}
-
-// dK, dV: one thread per key; loops over queries >= key.
-template <typename T, int HD>
-__global__ __launch_bounds__(64) void attn_bwd_kv_simt(const T* __restrict__ q, const T* __restrict__ k,
-                                                       const T* __restrict__ v, int64_t ldq, int64_t ldk,
-                                                       const T* __restrict__ dout, int64_t ldo,
-                                                       const float* __restrict__ lse, const float* __restrict__ Dg,
-                                                       T* dk, T* dv, int64_t ldd, int64_t lddk, int H, int S, int Sk,
-                                                       float scale, int causal) {
-    __shared__ float sq[kSimtTile][HD + 1];
-    __shared__ float sdo[kSimtTile][HD + 1];
-    __shared__ float sl[kSimtTile], sD[kSimtTile];
-    const int h = blockIdx.y, b = blockIdx.z;
-    const int kj = blockIdx.x * kSimtTile + threadIdx.x;
-    const int64_t tok0 = static_cast<int64_t>(b) * S, tok0k = static_cast<int64_t>(b) * Sk;
-    const int64_t hoff = static_cast<int64_t>(h) * HD;
-    const float* lse_bh = lse + (static_cast<int64_t>(b) * H + h) * S;
-    const float* D_bh = Dg + (static_cast<int64_t>(b) * H + h) * S;
-    float kv_[HD], vv[HD], dka[HD], dva[HD];
-    for (int d = 0; d < HD; ++d) {
-        kv_[d] = kj < Sk ? ld(k, (tok0k + kj) * ldk + hoff + d) : 0.0f;
-        vv[d] = kj < Sk ? ld(v, (tok0k + kj) * ldk + hoff + d) : 0.0f;
-        dka[d] = 0.0f;
-        dva[d] = 0.0f;
-    }
-    const int qstart = causal ? static_cast<int>(blockIdx.x * kSimtTile) : 0;
-    for (int q0 = qstart; q0 < S; q0 += kSimtTile) {
-        __syncthreads();
-        for (int e = threadIdx.x; e < kSimtTile * HD; e += 64) {
-            const int r = e / HD, d = e % HD;
-            const int qq = q0 + r;
-            sq[r][d] = qq < S ? ld(q, (tok0 + qq) * ldq + hoff + d) : 0.0f;
-            sdo[r][d] = qq < S ? ld(dout, (tok0 + qq) * ldo + hoff + d) : 0.0f;
-        }
-        if (threadIdx.x < kSimtTile) {
-            const int qq = q0 + threadIdx.x;
-            sl[threadIdx.x] = qq < S ? lse_bh[qq] : 0.0f;
-            sD[threadIdx.x] = qq < S ? D_bh[qq] : 0.0f;
-        }
-        __syncthreads();
-        if (kj >= Sk) continue;
-        for (int r = 0; r < kSimtTile; ++r) {
-            const int qq = q0 + r;
-            if (qq >= S) break;
-            if (causal && kj > qq) continue;
-            float sdot = 0.0f, dpd = 0.0f;
-            for (int d = 0; d < HD; ++d) {
-                sdot += sq[r][d] * kv_[d];
-                dpd += sdo[r][d] * vv[d];
-            }
-            const float p = expf(sdot * scale - sl[r]);
-            const float ds = p * (dpd - sD[r]);
-            for (int d = 0; d < HD; ++d) {
-                dva[d] += p * sdo[r][d];
-                dka[d] += ds * sq[r][d];
-            }
-        }
-    }
-    if (kj < Sk)
-        for (int d = 0; d < HD; ++d) {
-            st(dk, (tok0k + kj) * lddk + hoff + d, dka[d] * scale);
-            st(dv, (tok0k + kj) * lddk + hoff + d, dva[d]);
-        }
-}
-
-template <typename T, int HD>
-__global__ __launch_bounds__(64) void attn_bwd_q_simt(const T* __restrict__ q, const T* __restrict__ k,
-                                                      const T* __restrict__ v, int64_t ldq, int64_t ldk,
-                                                      const T* __restrict__ dout, int64_t ldo,
-                                                      const float* __restrict__ lse, const float* __restrict__ Dg, T* dq,
-                                                      int64_t ldd, int H, int S, int Sk, float scale, int causal) {
-    __shared__ float sk[kSimtTile][HD + 1];
-    __shared__ float sv[kSimtTile][HD + 1];
-    const int h = blockIdx.y, b = blockIdx.z;
-    const int qi = blockIdx.x * kSimtTile + threadIdx.x;
-    const int64_t tok0 = static_cast<int64_t>(b) * S, tok0k = static_cast<int64_t>(b) * Sk;
-    const int64_t hoff = static_cast<int64_t>(h) * HD;
-    float qv[HD], dov[HD], acc[HD];
-    for (int d = 0; d < HD; ++d) {
-        qv[d] = qi < S ? ld(q, (tok0 + qi) * ldq + hoff + d) : 0.0f;
-        dov[d] = qi < S ? ld(dout, (tok0 + qi) * ldo + hoff + d) : 0.0f;
-        acc[d] = 0.0f;
-    }
-    const float l = qi < S ? lse[(static_cast<int64_t>(b) * H + h) * S + qi] : 0.0f;
-    const float Dq = qi < S ? Dg[(static_cast<int64_t>(b) * H + h) * S + qi] : 0.0f;
-    const int kend = causal ? min(Sk, static_cast<int>((blockIdx.x + 1) * kSimtTile)) : Sk;
-    for (int k0 = 0; k0 < kend; k0 += kSimtTile) {
-        __syncthreads();
-        for (int e = threadIdx.x; e < kSimtTile * HD; e += 64) {
-            const int r = e / HD, d = e % HD;
-            const int key = k0 + r;
-            sk[r][d] = key < Sk ? ld(k, (tok0k + key) * ldk + hoff + d) : 0.0f;
-            sv[r][d] = key < Sk ? ld(v, (tok0k + key) * ldk + hoff + d) : 0.0f;
-        }
-        __syncthreads();
-        if (qi >= S) continue;
-        for (int r = 0; r < kSimtTile; ++r) {
-            const int key = k0 + r;
-            if (key >= Sk || (causal && key > qi)) break;
-            float sdot = 0.0f, dpd = 0.0f;
-            for (int d = 0; d < HD; ++d) {
-                sdot += qv[d] * sk[r][d];
-                dpd += dov[d] * sv[r][d];
-            }
-            const float p = expf(sdot * scale - l);
-            const float ds = p * (dpd - Dq);
-            for (int d = 0; d < HD; ++d) acc[d] += ds * sk[r][d];
-        }
-    }
-    if (qi < S)
-        for (int d = 0; d < HD; ++d) st(dq, (tok0 + qi) * ldd + hoff + d, acc[d] * scale);
-}
-
-// ---------------------------------------------------------------------------------------
-// Attention over a KV cache (decode): block (i, h, b) is query i of the S_new new tokens at
-// position start_pos + i; it attends to cache rows 0 .. start_pos + i.  Scores go to LDS
-// (one wave per key, lanes across head_dim, shuffle sums), then max, exp and sum in fixed
-// trees, then each thread accumulates one head_dim column over a strided key subset and the
-// subsets are added in a fixed order.  fp32 math; the row sums are deterministic.
-// ---------------------------------------------------------------------------------------
-template <typename T>
-__global__ __launch_bounds__(256) void attn_cached_k(const T* __restrict__ q, int64_t ldq, const T* __restrict__ kc,
-                                                     const T* __restrict__ vc, int64_t ldkv, int64_t bstride,
-                                                     T* __restrict__ o, int64_t ldo, int S_new, int start_pos, int hd,
-                                                     float scale) {
-    extern __shared__ float sm_dec[];
-    const int i = blockIdx.x, h = blockIdx.y, b = blockIdx.z;
-    const int L = start_pos + i + 1;
-    float* sc = sm_dec;           // [L] scores, then probabilities
-    float* red = sm_dec + L;      // [256]
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const T* qr = q + (static_cast<int64_t>(b) * S_new + i) * ldq + static_cast<int64_t>(h) * hd;
-    const T* kb = kc + static_cast<int64_t>(b) * bstride + static_cast<int64_t>(h) * hd;
-    const T* vb = vc + static_cast<int64_t>(b) * bstride + static_cast<int64_t>(h) * hd;
-    const float q0 = lane < hd ? ld(qr, lane) : 0.0f, q1 = lane + 64 < hd ? ld(qr, lane + 64) : 0.0f;
-    for (int j = wave; j < L; j += 4) {
-        const T* kr = kb + static_cast<int64_t>(j) * ldkv;
-        float p = (lane < hd ? q0 * ld(kr, lane) : 0.0f) + (lane + 64 < hd ? q1 * ld(kr, lane + 64) : 0.0f);
-#pragma unroll
-        for (int w = 32; w > 0; w >>= 1) p += __shfl_xor(p, w);
-        if (lane == 0) sc[j] = p * scale;
-    }
-    __syncthreads();
-    float m = -INFINITY;
-    for (int j = tid; j < L; j += 256) m = fmaxf(m, sc[j]);
-    red[tid] = m;
-    __syncthreads();
-    for (int w = 128; w > 0; w >>= 1) {
-        if (tid < w) red[tid] = fmaxf(red[tid], red[tid + w]);
-        __syncthreads();
-    }
-    m = red[0];
-    __syncthreads();
-    float sum = 0.0f;
-    for (int j = tid; j < L; j += 256) {
-        const float e = expf(sc[j] - m);
-        sc[j] = e;
-        sum += e;
-    }
-    red[tid] = sum;
-    __syncthreads();
-    for (int w = 128; w > 0; w >>= 1) {
-        if (tid < w) red[tid] += red[tid + w];
-        __syncthreads();
-    }
-    const float inv = 1.0f / red[0];
-    __syncthreads();
-    // thread t: column t % hd over keys j = t / hd, t / hd + G, ... (G = 256 / hd groups)
-    const int G = 256 / hd, d = tid % hd, g = tid / hd;
-    float acc = 0.0f;
-    if (g < G)
-        for (int j = g; j < L; j += G) acc += sc[j] * ld(vb + static_cast<int64_t>(j) * ldkv, d);
-    red[tid] = acc;
-    __syncthreads();
-    if (tid < hd) {
-        float t = 0.0f;
-        for (int u = 0; u < G; ++u) t += red[u * hd + tid];
-        st(o + (static_cast<int64_t>(b) * S_new + i) * ldo + static_cast<int64_t>(h) * hd, tid, t * inv);
-    }
-}
-
 bool a16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
 bool mfma_ok(const void* q, const void* k, const void* v, int64_t ldq, const void* o, int64_t ldo, int64_t hd) {
     return (hd == 64 || hd == 128) && ldq % 8 == 0 && ldo % 8 == 0 && a16(q) && a16(k) && a16(v) && a16(o) &&
            ldq < (int64_t{1} << 24) && ldo < (int64_t{1} << 24);  // 32-bit copy offsets (Rows64)
-}
-
-template <typename T>
-void fwd_simt(const void* q, const void* k, const void* v, int64_t ldq, int64_t ldk, void* o, int64_t ldo, float* lse,
-              int64_t B, int64_t H, int64_t S, int64_t Sk, int64_t hd, bool causal, float scale, hipStream_t s) {
-    const dim3 grid(static_cast<unsigned>((S + kSimtTile - 1) / kSimtTile), static_cast<unsigned>(H),
-                    static_cast<unsigned>(B));
-#define AIC_FWD_SIMT(HD_)                                                                                     \
-    hipLaunchKernelGGL((attn_fwd_simt<T, HD_>), grid, dim3(64), 0, s, static_cast<const T*>(q),                \
-                       static_cast<const T*>(k), static_cast<const T*>(v), ldq, ldk, static_cast<T*>(o), ldo, lse, \
-                       static_cast<int>(H), static_cast<int>(S), static_cast<int>(Sk), scale, causal ? 1 : 0)
-    if (hd == 16) AIC_FWD_SIMT(16);
-    else if (hd == 32) AIC_FWD_SIMT(32);
-    else if (hd == 64) AIC_FWD_SIMT(64);
-    else if (hd == 128) AIC_FWD_SIMT(128);
-    else AIC_THROW(NotImplemented, "attention: head_dim ", hd, " is not supported on this path");
-#undef AIC_FWD_SIMT
-    AIC_LAUNCH_CHECK("attn_fwd_simt");
-}
-
-template <typename T>
-void bwd_simt(const void* q, const void* k, const void* v, int64_t ldq, int64_t ldk, const void* dout, int64_t ldo,
-              const float* lse, const float* D, void* dq, int64_t ldd, void* dk, void* dv, int64_t lddk, int64_t B,
-              int64_t H, int64_t S, int64_t Sk, int64_t hd, bool causal, float scale, hipStream_t s) {
-    const dim3 grid(static_cast<unsigned>((S + kSimtTile - 1) / kSimtTile), static_cast<unsigned>(H),
-                    static_cast<unsigned>(B));
-    const dim3 gridk(static_cast<unsigned>((Sk + kSimtTile - 1) / kSimtTile), static_cast<unsigned>(H),
-                     static_cast<unsigned>(B));
-#define AIC_BWD_SIMT(HD_)                                                                                      \
-    do {                                                                                                        \
-        hipLaunchKernelGGL((attn_bwd_kv_simt<T, HD_>), gridk, dim3(64), 0, s, static_cast<const T*>(q),         \
-                           static_cast<const T*>(k), static_cast<const T*>(v), ldq, ldk,                        \
-                           static_cast<const T*>(dout), ldo, lse, D, static_cast<T*>(dk), static_cast<T*>(dv),   \
-                           ldd, lddk, static_cast<int>(H), static_cast<int>(S), static_cast<int>(Sk), scale,    \
-                           causal ? 1 : 0);                                                                      \
-        if (S > 0)                                                                                              \
-            hipLaunchKernelGGL((attn_bwd_q_simt<T, HD_>), grid, dim3(64), 0, s, static_cast<const T*>(q),       \
-                               static_cast<const T*>(k), static_cast<const T*>(v), ldq, ldk,                    \
-                               static_cast<const T*>(dout), ldo, lse, D, static_cast<T*>(dq), ldd,               \
-                               static_cast<int>(H), static_cast<int>(S), static_cast<int>(Sk), scale,           \
-                               causal ? 1 : 0);                                                                  \
-    } while (0)
-    if (hd == 16) AIC_BWD_SIMT(16);
-    else if (hd == 32) AIC_BWD_SIMT(32);
-    else if (hd == 64) AIC_BWD_SIMT(64);
-    else if (hd == 128) AIC_BWD_SIMT(128);
-    else AIC_THROW(NotImplemented, "attention: head_dim ", hd, " is not supported on this path");
-#undef AIC_BWD_SIMT
-    AIC_LAUNCH_CHECK("attn_bwd_simt");
 }
 
 }  // namespace
@@ -1213,10 +877,7 @@ void attn_fwd(const void* q, const void* k, const void* v, int64_t ld_qkv, void*
         AIC_LAUNCH_CHECK("attn_fwd_pipe");
         return;
     }
-    if (dt == DType::Float32) fwd_simt<float>(q, k, v, ld_qkv, ld_qkv, o, ld_o, lse, B, H, S, S, hd, causal, scale, s);
-    else if (dt == DType::BFloat16)
-        fwd_simt<bf16>(q, k, v, ld_qkv, ld_qkv, o, ld_o, lse, B, H, S, S, hd, causal, scale, s);
-    else AIC_THROW(DTypeMismatch, "attn_fwd: dtype must be f32 or bf16");
+    attn_fwd_qk(q, ld_qkv, k, v, ld_qkv, o, ld_o, lse, B, H, S, S, hd, causal, scale, dt, s);
 }
 
 void attn_bwd(const void* q, const void* k, const void* v, int64_t ld_qkv, const void* o, const void* dout,
@@ -1229,9 +890,9 @@ void attn_bwd(const void* q, const void* k, const void* v, int64_t ld_qkv, const
     AIC_CHECK(S < (1LL << 30) && B * S < (1LL << 31) && ((S + 127) / 128) * H * B < (1LL << 31), InvalidArgument,
               "attn_bwd: sequence too long");
     if (B == 0 || S == 0) return;
-    float* D = static_cast<float*>(stream_scratch(sizeof(float) * B * H * S, s));
     if (dt == DType::BFloat16 && mfma_ok(q, k, v, ld_qkv, dout, ld_o, hd) && ld_d % 8 == 0 && a16(dq) && a16(dk) &&
         a16(dv) && a16(o)) {
+        float* D = static_cast<float*>(stream_scratch(sizeof(float) * B * H * S, s));
         // the dQ kernel computes D = rowsum(dO * O) for its queries and writes it for dK/dV
         const float sl2 = scale * kLog2e;
         const dim3 grid(static_cast<unsigned>(((S + 127) / 128) * H * B));
@@ -1255,41 +916,7 @@ void attn_bwd(const void* q, const void* k, const void* v, int64_t ld_qkv, const
 #undef AIC_BWD_MFMA
         return;
     }
-    const int64_t waves = B * S * H;
-    const unsigned dgrid = static_cast<unsigned>((waves * 64 + 255) / 256);
-    const bool al16 = (reinterpret_cast<uintptr_t>(o) & 15u) == 0 && (reinterpret_cast<uintptr_t>(dout) & 15u) == 0;
-    if (dt == DType::BFloat16 && ld_o % 8 == 0 && al16 && (hd == 32 || hd == 64 || hd == 128)) {
-        const int64_t rpw = 64 / (hd / 8);  // rows per wave
-        const unsigned g8 = static_cast<unsigned>(((waves + rpw - 1) / rpw * 64 + 255) / 256);
-        const bf16* ob = static_cast<const bf16*>(o);
-        const bf16* db = static_cast<const bf16*>(dout);
-        if (hd == 128)
-            hipLaunchKernelGGL(attn_dot_v8_k<128>, dim3(g8), dim3(256), 0, s, ob, db, ld_o, D, B * S,
-                               static_cast<int>(H), static_cast<int>(S));
-        else if (hd == 64)
-            hipLaunchKernelGGL(attn_dot_v8_k<64>, dim3(g8), dim3(256), 0, s, ob, db, ld_o, D, B * S,
-                               static_cast<int>(H), static_cast<int>(S));
-        else
-            hipLaunchKernelGGL(attn_dot_v8_k<32>, dim3(g8), dim3(256), 0, s, ob, db, ld_o, D, B * S,
-                               static_cast<int>(H), static_cast<int>(S));
-    } else if (dt == DType::BFloat16)
-        hipLaunchKernelGGL(attn_dot_k<bf16>, dim3(dgrid), dim3(256), 0, s, static_cast<const bf16*>(o),
-                           static_cast<const bf16*>(dout), ld_o, D, B * S, static_cast<int>(H), static_cast<int>(S),
-                           static_cast<int>(hd));
-    else if (dt == DType::Float32)
-        hipLaunchKernelGGL(attn_dot_k<float>, dim3(dgrid), dim3(256), 0, s, static_cast<const float*>(o),
-                           static_cast<const float*>(dout), ld_o, D, B * S, static_cast<int>(H), static_cast<int>(S),
-                           static_cast<int>(hd));
-    else
-        AIC_THROW(DTypeMismatch, "attn_bwd: dtype must be f32 or bf16");
-    AIC_LAUNCH_CHECK("attn_dot");
-
-    if (dt == DType::Float32)
-        bwd_simt<float>(q, k, v, ld_qkv, ld_qkv, dout, ld_o, lse, D, dq, ld_d, dk, dv, ld_d, B, H, S, S, hd, causal,
-                        scale, s);
-    else
-        bwd_simt<bf16>(q, k, v, ld_qkv, ld_qkv, dout, ld_o, lse, D, dq, ld_d, dk, dv, ld_d, B, H, S, S, hd, causal,
-                       scale, s);
+    attn_bwd_qk(q, ld_qkv, k, v, ld_qkv, o, dout, ld_o, lse, dq, ld_d, dk, dv, ld_d, B, H, S, S, hd, causal, scale, dt, s);
     if (rope_cos) {  // the rotary embedding's adjoint as its own pass on these paths
         rope(dq, ld_d, B, S, H, hd, 0, rope_cos, rope_sin, true, dt, s);
         rope(dk, ld_d, B, S, H, hd, 0, rope_cos, rope_sin, true, dt, s);
@@ -1299,8 +926,7 @@ void attn_bwd(const void* q, const void* k, const void* v, int64_t ld_qkv, const
 // Queries and keys of different lengths (launch_flash_attention_forward/backward_gpu take
 // seq_len_q and seq_len_k, src/cuda/cuda_flash_attention.cuh:12-46): q, o, dO [B, Sq] token rows
 // of H heads (leading dimensions ld_q, ld_o), k, v [B, Sk] rows (ld_k); causal as the reference's
-// CPU path (src/ops/flash_attention.cpp:76-89, 170-260): query r sees keys c <= r.  The SIMT
-// kernels (fp32 math) for any dtype; lse [B, H, Sq].
+// CPU path (src/ops/flash_attention.cpp:76-89, 170-260): query r sees keys c <= r.  lse [B, H, Sq].
 void attn_fwd_qk(const void* q, int64_t ld_q, const void* k, const void* v, int64_t ld_k, void* o, int64_t ld_o,
                  float* lse, int64_t B, int64_t H, int64_t Sq, int64_t Sk, int64_t hd, bool causal, float scale,
                  DType dt, hipStream_t s) {
@@ -1310,10 +936,12 @@ void attn_fwd_qk(const void* q, int64_t ld_q, const void* k, const void* v, int6
               "attn_fwd: sequence too long");
     if (B == 0 || Sq == 0) return;
     AIC_CHECK(Sk > 0, InvalidArgument, "attn_fwd: no keys");
-    if (dt == DType::Float32) fwd_simt<float>(q, k, v, ld_q, ld_k, o, ld_o, lse, B, H, Sq, Sk, hd, causal, scale, s);
-    else if (dt == DType::BFloat16)
-        fwd_simt<bf16>(q, k, v, ld_q, ld_k, o, ld_o, lse, B, H, Sq, Sk, hd, causal, scale, s);
-    else AIC_THROW(DTypeMismatch, "attn_fwd: dtype must be f32 or bf16");
+    GenAttn a;
+    a.q = q; a.k = k; a.v = v; a.o_out = o; a.lse_out = lse;
+    a.ldq = ld_q; a.ldk = ld_k; a.ldo = ld_o;
+    a.B = B; a.H = H; a.Sq = Sq; a.Sk = a.kv_rows = Sk; a.hd = hd;
+    a.causal = causal; a.scale = scale;
+    attn_general_forward(a, dt, s);
 }
 
 void attn_bwd_qk(const void* q, int64_t ld_q, const void* k, const void* v, int64_t ld_k, const void* o,
@@ -1328,26 +956,13 @@ void attn_bwd_qk(const void* q, int64_t ld_q, const void* k, const void* v, int6
     if (B == 0) return;
     AIC_CHECK(Sk > 0, InvalidArgument, "attn_bwd: no keys");
     AIC_CHECK(dt == DType::Float32 || dt == DType::BFloat16, DTypeMismatch, "attn_bwd: dtype must be f32 or bf16");
-    // no queries: only the key kernel runs, and its empty query loop writes zero dK and dV
-    float* D = static_cast<float*>(stream_scratch(sizeof(float) * std::max<int64_t>(B * H * Sq, 1), s));
-    if (Sq > 0) {
-        const unsigned dgrid = static_cast<unsigned>((B * Sq * H * 64 + 255) / 256);
-        if (dt == DType::Float32)
-            hipLaunchKernelGGL(attn_dot_k<float>, dim3(dgrid), dim3(256), 0, s, static_cast<const float*>(o),
-                               static_cast<const float*>(dout), ld_o, D, B * Sq, static_cast<int>(H),
-                               static_cast<int>(Sq), static_cast<int>(hd));
-        else
-            hipLaunchKernelGGL(attn_dot_k<bf16>, dim3(dgrid), dim3(256), 0, s, static_cast<const bf16*>(o),
-                               static_cast<const bf16*>(dout), ld_o, D, B * Sq, static_cast<int>(H),
-                               static_cast<int>(Sq), static_cast<int>(hd));
-        AIC_LAUNCH_CHECK("attn_dot");
-    }
-    if (dt == DType::Float32)
-        bwd_simt<float>(q, k, v, ld_q, ld_k, dout, ld_o, lse, D, dq, ld_dq, dk, dv, ld_dkv, B, H, Sq, Sk, hd, causal,
-                        scale, s);
-    else
-        bwd_simt<bf16>(q, k, v, ld_q, ld_k, dout, ld_o, lse, D, dq, ld_dq, dk, dv, ld_dkv, B, H, Sq, Sk, hd, causal,
-                       scale, s);
+    GenAttn a;
+    a.q = q; a.k = k; a.v = v; a.o = o; a.dout = dout; a.lse = lse;
+    a.dq = dq; a.dk = dk; a.dv = dv;
+    a.ldq = ld_q; a.ldk = ld_k; a.ldo = ld_o; a.ld_dq = ld_dq; a.ld_dkv = ld_dkv;
+    a.B = B; a.H = H; a.Sq = Sq; a.Sk = a.kv_rows = Sk; a.hd = hd;
+    a.causal = causal; a.scale = scale;
+    attn_general_backward(a, dt, s);
 }
 
 void attn_cached(const void* q, int64_t ldq, const void* kc, const void* vc, int64_t ldkv, int64_t cache_rows, void* o,
@@ -1359,30 +974,12 @@ void attn_cached(const void* q, int64_t ldq, const void* kc, const void* vc, int
     AIC_CHECK(start_pos + S_new <= cache_rows && start_pos + S_new <= 16384, InvalidArgument,
               "attn_cached: the cache holds ", cache_rows, " positions (at most 16384), needed ", start_pos + S_new);
     if (B == 0 || S_new == 0) return;
-    const dim3 grid(static_cast<unsigned>(S_new), static_cast<unsigned>(H), static_cast<unsigned>(B));
-    const size_t lds = sizeof(float) * static_cast<size_t>(start_pos + S_new + 256);
-    const int64_t bstride = cache_rows * ldkv;
-    static bool configured = false;  // allow the scores of up to 16384 positions in LDS
-    if (!configured) {
-        AIC_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_cached_k<bf16>),
-                                          hipFuncAttributeMaxDynamicSharedMemorySize, 96 * 1024));
-        AIC_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_cached_k<float>),
-                                          hipFuncAttributeMaxDynamicSharedMemorySize, 96 * 1024));
-        configured = true;
-    }
-    if (dt == DType::BFloat16)
-        hipLaunchKernelGGL(attn_cached_k<bf16>, grid, dim3(256), lds, s, static_cast<const bf16*>(q), ldq,
-                           static_cast<const bf16*>(kc), static_cast<const bf16*>(vc), ldkv, bstride,
-                           static_cast<bf16*>(o), ldo, static_cast<int>(S_new), static_cast<int>(start_pos),
-                           static_cast<int>(hd), scale);
-    else if (dt == DType::Float32)
-        hipLaunchKernelGGL(attn_cached_k<float>, grid, dim3(256), lds, s, static_cast<const float*>(q), ldq,
-                           static_cast<const float*>(kc), static_cast<const float*>(vc), ldkv, bstride,
-                           static_cast<float*>(o), ldo, static_cast<int>(S_new), static_cast<int>(start_pos),
-                           static_cast<int>(hd), scale);
-    else
-        AIC_THROW(DTypeMismatch, "attn_cached: dtype must be f32 or bf16");
-    AIC_LAUNCH_CHECK("attn_cached");
+    GenAttn a;
+    a.q = q; a.k = kc; a.v = vc; a.o_out = o;
+    a.ldq = ldq; a.ldk = ldkv; a.ldo = ldo;
+    a.B = B; a.H = H; a.Sq = S_new; a.Sk = start_pos + S_new; a.kv_rows = cache_rows; a.hd = hd;
+    a.causal = true; a.start = start_pos; a.scale = scale;
+    attn_general_forward(a, dt, s);
 }
 
 }  // namespace aic::hip

@@ -133,6 +133,23 @@ void attn_bwd_qk(const void* q, int64_t ld_q, const void* k, const void* v, int6
                  const void* dout, int64_t ld_o, const float* lse, void* dq, int64_t ld_dq, void* dk, void* dv,
                  int64_t ld_dkv, int64_t B, int64_t H, int64_t Sq, int64_t Sk, int64_t hd, bool causal, float scale,
                  DType dt, hipStream_t s);
+// The kernels behind attn_fwd_qk / attn_bwd_qk / attn_cached and behind the shapes and types that
+// attn_fwd / attn_bwd's own kernels do not take (attention_general.hip).  Row b * Sq + s of q, o,
+// dout, dq; row b * kv_rows + s of k, v, dk, dv; causal: query r sees the keys c <= r + start.
+struct GenAttn {
+    const void *q = nullptr, *k = nullptr, *v = nullptr;
+    void* o_out = nullptr;                            // forward
+    float* lse_out = nullptr;                         // forward, nullable
+    const void *o = nullptr, *dout = nullptr;         // backward
+    const float* lse = nullptr;                       // backward
+    void *dq = nullptr, *dk = nullptr, *dv = nullptr;  // backward
+    int64_t ldq = 0, ldk = 0, ldo = 0, ld_dq = 0, ld_dkv = 0;
+    int64_t B = 0, H = 0, Sq = 0, Sk = 0, kv_rows = 0, hd = 0, start = 0;
+    bool causal = false;
+    float scale = 1.0f;
+};
+void attn_general_forward(const GenAttn& a, DType dt, hipStream_t s);
+void attn_general_backward(const GenAttn& a, DType dt, hipStream_t s);
 // Queries of S_new new tokens (rows of q, [B*S_new] x ldq) at positions start_pos.. against a
 // KV cache kc / vc ([B][cache_rows][ldkv], positions 0 .. start_pos+S_new-1 filled), causal.
 void attn_cached(const void* q, int64_t ldq, const void* kc, const void* vc, int64_t ldkv, int64_t cache_rows, void* o,

@@ -1,0 +1,106 @@
+"""The general attention kernels (csrc/kernels/attention_general.hip) where their tiling can go
+wrong: lengths around the 16-row tiles and 32-row blocks, one query, groups shared by several
+waves, head_dim 16 to 128, and rows whose leading dimension or base rules out 16-byte loads.
+Each head against the oracle's restatement of the CPU path (src/ops/flash_attention.cpp:32-260)
+within the bounds that the launcher tests use for the same entries: fp32 sums over up to 2000
+keys, and one bf16 rounding of the outputs."""
+import numpy as np
+import pytest
+
+torch = pytest.importorskip("torch")
+
+pytestmark = pytest.mark.gpu
+
+from autonomousaicore_amd import _lib  # noqa: E402
+from tests.gpu_util import bf16_round, call, host, rel, stream  # noqa: E402
+
+F32, BF16 = _lib.AIC_F32, _lib.AIC_BF16
+
+
+@pytest.fixture(scope="module", autouse=True)
+def _gpu():
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    torch.cuda.set_device(0)
+
+
+# (B, H, Sq, Sk, D, causal, pad, shift): rows of H * D + pad elements from an address shifted by
+# `shift` elements
+CASES = [(1, 1, 1, 1, 64, False, 0, 0), (1, 2, 1, 2000, 128, False, 0, 0), (2, 3, 16, 32, 32, True, 0, 0),
+         (1, 2, 17, 33, 16, False, 0, 0), (2, 2, 33, 31, 128, True, 8, 0), (1, 3, 47, 65, 64, False, 3, 0),
+         (1, 2, 31, 97, 128, True, 0, 1), (3, 4, 200, 130, 64, True, 8, 0), (1, 1, 5, 700, 16, False, 1, 3)]
+
+
+@pytest.mark.parametrize("dt", [F32, BF16])
+@pytest.mark.parametrize("B,H,Sq,Sk,D,causal,pad,shift", CASES)
+def test_attention_tile_edges(orc, dt, B, H, Sq, Sk, D, causal, pad, shift):
+    rng = np.random.default_rng(Sq * 7 + Sk * 3 + D + pad)
+    t, ld = torch.float32 if dt == F32 else torch.bfloat16, H * D + pad
+
+    def rows(n, fill=None):
+        """A [n, ld] matrix of its own, `shift` elements into its storage, between guard values."""
+        buf = torch.full((n * ld + shift + 16,), 7.0, dtype=t, device="cuda")
+        x = buf[shift:shift + n * ld].view(n, ld)
+        if fill is not None:
+            a = fill.standard_normal((n, ld)).astype(np.float32)
+            x.copy_(torch.from_numpy(a if dt == F32 else bf16_round(a)).to(t))
+        return buf, x
+
+    (_, q), (_, k), (_, v), (_, do) = rows(B * Sq, rng), rows(B * Sk, rng), rows(B * Sk, rng), rows(B * Sq, rng)
+    (bo, o), (bdq, dq), (bdk, dk), (bdv, dv) = rows(B * Sq), rows(B * Sq), rows(B * Sk), rows(B * Sk)
+    lse = torch.empty((B, H, Sq), dtype=torch.float32, device="cuda")
+    shape = (B, H, Sq, Sk, D, int(causal), 1.0 / np.sqrt(D), dt, stream())
+    p = lambda x: x.data_ptr()  # noqa: E731
+    call("aic_hip_attn_fwd_qk", p(q), ld, p(k), p(v), ld, p(o), ld, p(lse), *shape)
+    call("aic_hip_attn_bwd_qk", p(q), ld, p(k), p(v), ld, p(o), p(do), ld, p(lse), p(dq), ld, p(dk), p(dv), ld, *shape)
+
+    def heads(x, S):
+        return np.ascontiguousarray(host(x)[:, :H * D].reshape(B, S, H, D).transpose(0, 2, 1, 3).reshape(B * H, S, D))
+
+    Q, K, V, O, DO = heads(q, Sq), heads(k, Sk), heads(v, Sk), heads(o, Sq), heads(do, Sq)
+    o_ref, lse_ref = orc.flash_fwd(Q, K, V, causal)
+    L = host(lse).reshape(B * H, Sq)
+    assert np.max(np.abs(L - lse_ref)) < (2e-5 if dt == F32 else 1e-3)
+    assert rel(O, o_ref) < (2e-6 if dt == F32 else 4e-3)
+    tol = 2e-5 if dt == F32 else 8e-3
+    for name, got, ref in zip("q k v".split(), (heads(dq, Sq), heads(dk, Sk), heads(dv, Sk)),
+                              orc.flash_bwd(Q, K, V, O, DO, L, causal)):
+        # one key: dS = P (dP - D) cancels exactly in the reference; then the bound is absolute
+        assert rel(got, ref) < tol or np.max(np.abs(got - ref)) < tol, name
+    for buf, x in ((bo, o), (bdq, dq), (bdk, dk), (bdv, dv)):  # nothing outside the heads was written
+        inside = np.zeros(buf.numel(), bool)
+        inside[shift:shift + x.numel()].reshape(x.shape)[:, :H * D] = True
+        assert np.all(host(buf)[~inside] == 7.0)
+
+
+@pytest.mark.parametrize("dt", [F32, BF16])
+def test_attention_infinities_stay_where_they_are_seen(dt):
+    """Causal attention over 37 tokens whose last value row holds an infinity and whose last query
+    and key rows are NaN: only the last query's output, and no other row's gradient of the keys
+    and queries before it, may show them (the tiles give hidden rows weight zero, and zero times
+    an infinity is NaN)."""
+    t = torch.float32 if dt == F32 else torch.bfloat16
+    S, D = 37, 64
+    g = torch.Generator(device="cuda").manual_seed(3)
+    q, k, v, do = (torch.randn((S, D), generator=g, device="cuda").to(t) for _ in range(4))
+
+    def run(q, k, v, do):
+        o, lse = torch.empty_like(q), torch.empty((1, 1, S), device="cuda")
+        dq, dk, dv = (torch.empty_like(q) for _ in range(3))
+        shape = (1, 1, S, S, D, 1, 0.125, dt, stream())
+        p = [x.data_ptr() for x in (q, k, v, o, lse, do, dq, dk, dv)]
+        call("aic_hip_attn_fwd_qk", p[0], D, p[1], p[2], D, p[3], D, p[4], *shape)
+        call("aic_hip_attn_bwd_qk", p[0], D, p[1], p[2], D, p[3], p[5], D, p[4], p[6], D, p[7], p[8], D, *shape)
+        return [host(x) for x in (o, dq)]
+
+    clean = run(q, k, v, do)
+    v[S - 1, 5] = float("inf")
+    dirty = run(q, k, v, do)
+    assert np.isinf(dirty[0][S - 1, 5]) and np.all(np.isfinite(np.delete(dirty[0][S - 1], 5)))
+    k[S - 1], q[S - 1] = float("nan"), float("nan")
+    worse = run(q, k, v, do)
+    # the last 16-row tile's sums are formed row by row there: equal up to the order of the sums
+    tol = 1e-5 if dt == F32 else 8e-3
+    for got in (dirty, worse):
+        for a, b in zip(got, clean):
+            assert rel(a[:S - 1], b[:S - 1]) < tol
