@@ -408,7 +408,8 @@ __global__ __launch_bounds__(512) void attn_general_fwd(const Args<T> p) {
         }
     }
     if (p.split > 1) {
-        // every wave of the block reaches the barrier; part 0 adds the group's partial sums
+        // every wave of the block reaches the barriers; the group's waves add the partial sums of
+        // a share of the head columns each, part 0 collects them
         wait_lds();
         constexpr int STAT = HD / 16 * RT * 1024;
         park<HD, RT>(region, acc);
@@ -418,27 +419,40 @@ __global__ __launch_bounds__(512) void attn_general_fwd(const Args<T> p) {
             reinterpret_cast<float*>(region + STAT)[(RT + r) * 64 + lane] = l[r];
         }
         __syncthreads();
-        if (part != 0) return;
+        char* group = gen_lds + (wave - part) * p.region;
 #pragma unroll
         for (int r = 0; r < RT; ++r) {
-            float mx = m[r];
-            for (int w = 1; w < p.split; ++w)
-                mx = fmaxf(mx, reinterpret_cast<const float*>(region + w * p.region + STAT)[r * 64 + lane]);
+            float pm[8], mx = -INFINITY;
+#pragma unroll
+            for (int w = 0; w < 8; ++w)
+                if (w < p.split) {
+                    pm[w] = reinterpret_cast<const float*>(group + w * p.region + STAT)[r * 64 + lane];
+                    mx = fmaxf(mx, pm[w]);
+                }
             const float base = mx == -INFINITY ? 0.0f : mx;
-            const float f0 = exp_of<T>(m[r] - base);
-            l[r] *= f0;
+            l[r] = 0.0f;
 #pragma unroll
-            for (int dt = 0; dt < HD / 16; ++dt) acc[dt][r] *= f0;
-            for (int w = 1; w < p.split; ++w) {
-                const char* o = region + w * p.region;
-                const float f = exp_of<T>(reinterpret_cast<const float*>(o + STAT)[r * 64 + lane] - base);
-                l[r] += f * reinterpret_cast<const float*>(o + STAT)[(RT + r) * 64 + lane];
-#pragma unroll
-                for (int dt = 0; dt < HD / 16; ++dt)
-                    acc[dt][r] += f * *reinterpret_cast<const f32x4*>(o + ((dt * RT + r) * 64 + lane) * 16);
-            }
+            for (int w = 0; w < 8; ++w)
+                if (w < p.split) {
+                    pm[w] = exp_of<T>(pm[w] - base);
+                    l[r] += pm[w] * reinterpret_cast<const float*>(group + w * p.region + STAT)[(RT + r) * 64 + lane];
+                }
             m[r] = mx;
+            for (int dt = part; dt < HD / 16; dt += p.split) {
+                f32x4 t = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+                for (int w = 0; w < 8; ++w)
+                    if (w < p.split)
+                        t += pm[w] * *reinterpret_cast<const f32x4*>(group + w * p.region + ((dt * RT + r) * 64 + lane) * 16);
+                *reinterpret_cast<f32x4*>(group + ((dt * RT + r) * 64 + lane) * 16) = t;
+            }
         }
+        __syncthreads();
+        if (part != 0) return;
+#pragma unroll
+        for (int dt = 0; dt < HD / 16; ++dt)
+#pragma unroll
+            for (int r = 0; r < RT; ++r) acc[dt][r] = *reinterpret_cast<const f32x4*>(region + ((dt * RT + r) * 64 + lane) * 16);
     }
 #pragma unroll
     for (int r = 0; r < RT; ++r) {
@@ -726,6 +740,18 @@ __global__ __launch_bounds__(256) void attn_general_dkdv(const Args<T> p) {
     }
 }
 
+// V: the copied vector type; n vectors per d columns.
+template <typename V>
+__global__ __launch_bounds__(256) void kv_append_k(const V* __restrict__ qkv, V* kc, V* vc, int64_t rows, int S, int n,
+                                                   int64_t cache_rows, int64_t start) {
+    const int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+    if (i >= rows * 2 * n) return;
+    const int64_t t = i / (2 * n);
+    const int c = static_cast<int>(i % (2 * n));
+    const int64_t row = t / S * cache_rows + start + t % S;
+    (c < n ? kc : vc)[row * n + (c < n ? c : c - n)] = qkv[t * 3 * n + n + c];
+}
+
 enum Kind { kFwd, kDq, kDkDv };
 
 bool rows16(const void* p, int64_t ld, size_t es) {
@@ -851,6 +877,25 @@ void attn_general_backward(const GenAttn& a, DType dt, hipStream_t s) {
     if (dt == DType::Float32) bwd<float>(a, s);
     else if (dt == DType::BFloat16) bwd<bf16>(a, s);
     else AIC_THROW(DTypeMismatch, "attention: dtype must be f32 or bf16");
+}
+
+void kv_append(const void* qkv, void* kc, void* vc, int64_t B, int64_t S, int64_t d, int64_t cache_rows,
+               int64_t start_pos, DType dt, hipStream_t s) {
+    const int64_t rows = B * S, bytes = d * static_cast<int64_t>(dtype_size(dt));
+    if (rows == 0) return;
+    auto run = [&](auto v) {
+        using V = decltype(v);
+        const int64_t n = bytes / static_cast<int64_t>(sizeof(V));
+        const int64_t grid = (rows * 2 * n + 255) / 256;
+        AIC_CHECK(grid < (int64_t{1} << 31) && S < (int64_t{1} << 31), InvalidArgument, "kv_append: too many tokens");
+        hipLaunchKernelGGL(kv_append_k<V>, dim3(static_cast<unsigned>(grid)), dim3(256), 0, s, static_cast<const V*>(qkv),
+                           static_cast<V*>(kc), static_cast<V*>(vc), rows, static_cast<int>(S), static_cast<int>(n),
+                           cache_rows, start_pos);
+        AIC_LAUNCH_CHECK("kv_append");
+    };
+    auto fits = [&](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; };
+    if (bytes % 16 == 0 && fits(qkv) && fits(kc) && fits(vc)) run(uint4{});
+    else run(uint16_t{});
 }
 
 }  // namespace aic::hip

@@ -42,6 +42,25 @@ __device__ __forceinline__ float bf2f(bf16 h) {
     return __uint_as_float(static_cast<uint32_t>(__builtin_bit_cast(uint16_t, h)) << 16);
 }
 
+// Eight INT4 values (one packed dword: element e in bits 4e..4e+3, two's complement) times the
+// scale s, rounded to bf16.  With u = q + 8 (the nibble xor 8), fma(u, s, -8 s) is one rounding
+// of the exact q s, so every value equals the standalone dequantization's bf16(q * s).
+__device__ __forceinline__ uint4 q4_dequant8(uint32_t w, float s, float ns8) {
+    const uint32_t x = w ^ 0x88888888u;
+    uint32_t lo = x & 0x0f0f0f0fu, hi = (x >> 4) & 0x0f0f0f0fu;  // elements 0,2,4,6 and 1,3,5,7
+    // opaque to the optimizer, which would otherwise fold the masks into one bit-field extract
+    // per element instead of converting bytes with v_cvt_f32_ubyte0..3
+    asm volatile("" : "+v"(lo), "+v"(hi));
+    float v[8];
+#pragma unroll
+    for (int b = 0; b < 4; ++b) {
+        v[2 * b] = fmaf(static_cast<float>((lo >> (8 * b)) & 0xffu), s, ns8);
+        v[2 * b + 1] = fmaf(static_cast<float>((hi >> (8 * b)) & 0xffu), s, ns8);
+    }
+    return make_uint4(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]), pack_bf16x2(v[4], v[5]),
+                      pack_bf16x2(v[6], v[7]));
+}
+
 // Generic element load/store with fp32 compute.
 template <typename T> __device__ __forceinline__ float ld(const T* p, int64_t i);
 template <> __device__ __forceinline__ float ld<float>(const float* p, int64_t i) { return p[i]; }

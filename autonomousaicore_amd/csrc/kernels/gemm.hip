@@ -317,6 +317,28 @@ void gemm_q4(const GemmArgs& a, hipStream_t s) {
                       : gemm_impl::launch_dma_q4<128, 128, 64, 2, false, bf16>(a, s);
     }
 }
+
+// Few rows of x W^T: the kernel of gemm_skinny.hip (its low-rank term separately where the kernel
+// cannot take it).  False: not its shape.
+bool try_skinny(const GemmArgs& a, hipStream_t s) {
+    // From 17 rows on the tiles' padding shrinks and the skinny kernel's blocks read x again and
+    // again: a dense bf16 product stays on it only up to 4 M weights (64 rows: 2048x2048 11.5 us
+    // against 14.2 on split tiles, 768x2048 11.4 against 14.7, 6144x2048 20.4 against 18.4, 32 rows:
+    // 2048x5632 16.7 against 12.5, 11264x2048 18.7 against 15.8).
+    if (a.M > 16 && !a.Bq && a.ab == DType::BFloat16 && a.N * a.K > (int64_t{1} << 22)) return false;
+    SkinnyArgs q;
+    q.g = a;
+    if (gemm_skinny_eligible(q)) {
+        gemm_skinny(q, s);
+        return true;
+    }
+    if (a.r2 == 0 || a.rope_cos || a.glu_f > 0) return false;
+    q.g.r2 = 0;
+    if (!gemm_skinny_eligible(q)) return false;
+    gemm_skinny(q, s);
+    rank_term_separately(a, s);
+    return true;
+}
 }  // namespace
 
 void gemm(const GemmArgs& a, hipStream_t s) {
@@ -356,6 +378,7 @@ void gemm(const GemmArgs& a, hipStream_t s) {
         AIC_CHECK(a.rope_sin && a.rope_hd > 0 && a.rope_hd % 2 == 0 && a.rope_cols % a.rope_hd == 0 &&
                       a.rope_cols <= a.N && a.rope_seq > 0 && a.M % a.rope_seq == 0 && a.beta == 0.0f && !a.R,
                   InvalidArgument, "GEMM rotary epilogue: bad rope arguments");
+        if (try_skinny(a, s)) return;
         // in the epilogue: bf16 output on full 256x256 tiles, for the eight-wave plain path heads of
         // 128 (split in halves by the 64-column wave sub-tiles, exchanged through LDS) or 64 (one
         // per wave sub-tile), for the four-wave INT4 path heads of 128 (one per wave sub-tile,
@@ -390,6 +413,7 @@ void gemm(const GemmArgs& a, hipStream_t s) {
     if (a.glu_f > 0) {
         AIC_CHECK(a.N == 2 * a.glu_f && a.glu_out && a.ld_glu >= a.glu_f && a.beta == 0.0f && !a.R && !a.rope_cos,
                   InvalidArgument, "GEMM SwiGLU epilogue: bad arguments");
+        if (try_skinny(a, s)) return;
         // in the epilogue: bf16 x W^T on full 256x256 tiles of the eight-wave plain path, or of the
         // four-wave INT4 path (also after its low-rank term, whose segments follow the pairing)
         const bool tiles = a.transB && !a.transA && a.c == DType::BFloat16 && a.M % 256 == 0 && a.glu_f % 128 == 0 &&
@@ -430,6 +454,7 @@ void gemm(const GemmArgs& a, hipStream_t s) {
             return;
         }
     }
+    if (try_skinny(a, s)) return;
     if (a.Bq) {
         gemm_q4(a, s);
         return;

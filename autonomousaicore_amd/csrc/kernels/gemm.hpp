@@ -92,6 +92,24 @@ bool gemm_mfma_eligible(const GemmArgs& a);
 bool gemm_q4_eligible(const GemmArgs& a);
 bool gemm_dma_eligible(const GemmArgs& a);
 void gemm(const GemmArgs& a, hipStream_t stream);
+// Products of at most kSkinnyRows rows with W [N][K] (transA 0, transB 1; gemm_skinny.hip), with the
+// epilogues of GemmArgs (not dglu, not sq) at any size, and optionally: A's rows normalised first
+// (norm_w, [K]: op(A) = A / rms(A) * w, at most 16 rows); the k and v columns of a q/k/v product
+// also stored to the KV cache (kc, vc: [batch][kv_rows][d]; row m is position rope_start + m %
+// rope_seq of sequence m / rope_seq); skip_c: only glu_out is written.  gemm() runs them on this
+// path by itself where it can.
+constexpr int64_t kSkinnyRows = 64;
+struct SkinnyArgs {
+    GemmArgs g;
+    const float* norm_w = nullptr;
+    float norm_eps = 0.0f;
+    void* kc = nullptr;
+    void* vc = nullptr;
+    int64_t kv_rows = 0;
+    bool skip_c = false;
+};
+bool gemm_skinny_eligible(const SkinnyArgs& q);
+void gemm_skinny(const SkinnyArgs& q, hipStream_t stream);
 // Independent products in one launch when they share the kernel configuration (transposes,
 // dtypes, alpha, beta; no residual or low-rank term; up to 8), so that their tiles fill the
 // chip together instead of each product's last partial round; otherwise one gemm() each.

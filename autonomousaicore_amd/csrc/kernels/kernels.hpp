@@ -156,6 +156,11 @@ void attn_cached(const void* q, int64_t ldq, const void* kc, const void* vc, int
                  int64_t ldo, int64_t B, int64_t H, int64_t S_new, int64_t start_pos, int64_t hd, float scale, DType dt,
                  hipStream_t s);
 
+// The k and v columns of q/k/v rows qkv [B*S][3d] into the KV cache (kc, vc: [B][cache_rows][d]) at
+// positions start_pos ...
+void kv_append(const void* qkv, void* kc, void* vc, int64_t B, int64_t S, int64_t d, int64_t cache_rows,
+               int64_t start_pos, DType dt, hipStream_t s);
+
 // Optimizer tail (optim.hip)
 struct OptimCtl;  // = aic_optim_ctl (include/aic_hip.h)
 void grad_sqnorm_multi(const float* const* grads, const int64_t* sizes, int count, double* sqnorm, int* nonfinite,

@@ -58,7 +58,9 @@ bool fused_q4(int transW, int64_t M, int64_t N, int64_t K, float alpha, const vo
     a.Bscale = scales;
     a.scale_t = scale_t;
     a.group = hip::int4_group(N * K, group);
-    if (!hip::gemm_q4_eligible(a)) return false;
+    hip::SkinnyArgs few;
+    few.g = a;
+    if (!hip::gemm_q4_eligible(a) && !hip::gemm_skinny_eligible(few)) return false;
     hip::gemm(a, s);
     return true;
 }

@@ -79,16 +79,26 @@ struct SqOut {
     int64_t cap = 0;
 };
 
-void gemm(Profiler& prof, int ta, int tb, int64_t M, int64_t N, int64_t K, const void* A, int64_t lda,
+// Beside a product of few rows (hip::SkinnyArgs): RMSNorm of its input, the KV cache's new rows,
+// whether only the activation of a gate/up product is wanted.
+struct Decode {
+    const float* norm_w = nullptr;
+    float eps = 0.0f;
+    void* kc = nullptr;
+    void* vc = nullptr;
+    int64_t kv_rows = 0;
+    bool skip_c = false;
+};
+
+// False: `dec` was given and the product is not one that takes it (nothing was launched).
+bool gemm(Profiler& prof, int ta, int tb, int64_t M, int64_t N, int64_t K, const void* A, int64_t lda,
           const void* B, int64_t ldb, void* C, int64_t ldc, DType ab, DType c, hipStream_t s, const void* R = nullptr,
           int64_t ldr = 0, float beta = 0.0f, float alpha = 1.0f, const LowRank* lr = nullptr, Q4B q4 = {},
-          RopeOut rope = {}, GluOut glu = {}, DGlu dglu = {}, SqOut sq = {}) {
+          RopeOut rope = {}, GluOut glu = {}, DGlu dglu = {}, SqOut sq = {}, const Decode* dec = nullptr) {
     const double es = static_cast<double>(dtype_size(ab)), ec = static_cast<double>(dtype_size(c));
     const double kr = lr ? static_cast<double>(lr->r2) : 0.0;
     // INT4 operand: half a byte per weight plus one fp16 scale per group
     const double bbytes = q4.packed ? 0.5 * N * K + 2.0 * N * K / static_cast<double>(q4.group) : es * N * K;
-    auto scope = prof.scope(ta ? kGemmWgrad : (tb ? kGemmFwd : kGemmDgrad), 2.0 * M * N * (K + kr),
-                            es * M * K + bbytes + ec * M * N * (R ? 2 : 1), s);
     hip::GemmArgs a;
     a.transA = ta;
     a.transB = tb;
@@ -144,7 +154,22 @@ void gemm(Profiler& prof, int ta, int tb, int64_t M, int64_t N, int64_t K, const
     a.sq_part = sq.part;
     a.sq_nf = sq.nf;
     a.sq_cap = sq.cap;
-    hip::gemm(a, s);
+    hip::SkinnyArgs few;
+    if (dec) {
+        few.g = a;
+        few.norm_w = dec->norm_w;
+        few.norm_eps = dec->eps;
+        few.kc = dec->kc;
+        few.vc = dec->vc;
+        few.kv_rows = dec->kv_rows;
+        few.skip_c = dec->skip_c;
+        if (!hip::gemm_skinny_eligible(few)) return false;
+    }
+    auto scope = prof.scope(ta ? kGemmWgrad : (tb ? kGemmFwd : kGemmDgrad), 2.0 * M * N * (K + kr),
+                            es * M * K + bbytes + ec * M * N * (R ? 2 : 1), s);
+    if (dec) hip::gemm_skinny(few, s);
+    else hip::gemm(a, s);
+    return true;
 }
 
 // Weight gradients dW_i = A_i^T B_i (fp32 out) of independent products in one launch.
@@ -1301,18 +1326,15 @@ void TransformerLM::forward_step(const int64_t* ids, int64_t B, int64_t S, int64
     auto f32 = [&](int64_t elems) -> DeviceBuffer& {
         return workspace(slot++, sizeof(float) * static_cast<size_t>(elems));
     };
-    auto at = [&](const DeviceBuffer& b, int64_t elem) {
-        return static_cast<void*>(static_cast<char*>(b.get()) + es * static_cast<size_t>(elem));
-    };
     const bool moe = cfg_.num_experts > 0, ql = lora();
     const int64_t r = cfg_.lora_rank;
     const float lsc = ql ? cfg_.lora_alpha / static_cast<float>(r) : 0.0f;
     DeviceBuffer &xa = act(T * d), &xb = act(T * d), &h = act(T * d), &qkv = act(T * 3 * d), &ob = act(T * d),
                  &x1 = act(T * d), &gu = act(moe ? 0 : T * 2 * f), &am = act(moe ? 0 : T * f), &rr = f32(T),
                  &lse = f32(start_pos == 0 ? T * H : 0), &xs = act(ql ? T * 7 * r : 0);
-    // QLoRA base projections as in the training step: in-GEMM INT4 operands, or dequantized
-    // stack by stack into a scratch buffer (fp32 operands, or fewer than 8 rows)
-    const bool q4f = ql && q4_fused_ && T >= 8;
+    // QLoRA base projections as in-GEMM INT4 operands, or (fp32) dequantized stack by stack into a
+    // scratch buffer
+    const bool q4f = ql && q4_fused_;
     DeviceBuffer& wbuf = act(ql && !q4f ? std::max(3 * d * d, 2 * f * d) : 0);
     auto wbase = [&](const Layer& ly, int64_t off, int j0, int j1) -> const void* {
         if (!ql) return WB(off);
@@ -1322,65 +1344,82 @@ void TransformerLM::forward_step(const int64_t* ids, int64_t B, int64_t S, int64
     auto wq = [&](const Layer& ly, int j0) -> Q4B {
         return q4f ? Q4B{q4_ + ly.pk[j0], static_cast<const uint16_t*>(q4s_) + ly.sc[j0], cfg_.quant_group} : Q4B{};
     };
+    // A projection of RMSNorm(x) (norm: its weight) or of x itself.  With few tokens the product's
+    // blocks normalise the rows themselves, as long as that reads less than about 8 MB again
+    // (each block of 16 or 32 weight rows does); otherwise the norm runs once, before the first product that
+    // needs its rows.  W is called at most once, and only for the product that runs.
+    const float* normed = nullptr;  // the norm whose rows h holds
+    auto proj = [&](const void* in, const float* norm, int64_t N, int64_t K, auto&& weight, void* C, DType c, const void* R,
+                    float alpha, const LowRank* lr, Q4B q4, RopeOut rope, GluOut glu, Decode dec) {
+        const void* w = weight();
+        const int64_t again = static_cast<int64_t>(es) * T * K * (N / (rope.cos || glu.out || N > 16384 ? 32 : 16));
+        if (T <= 16 && norm && again <= (int64_t{8} << 20)) {
+            dec.norm_w = norm;
+            dec.eps = eps;
+            if (gemm(prof_, 0, 1, T, N, K, in, K, w, K, C, N, dt, c, s, R, N, 0.0f, alpha, lr, q4, rope, glu, {}, {}, &dec))
+                return true;
+            dec.norm_w = nullptr;
+        }
+        if (norm && normed != norm) {
+            hip::rmsnorm_fwd(in, K, norm, h.get(), K, rr.as<float>(), T, K, eps, dt, s);
+            normed = norm;
+        }
+        const void* A = norm ? h.get() : in;
+        if ((dec.kc || dec.skip_c) &&
+            gemm(prof_, 0, 1, T, N, K, A, K, w, K, C, N, dt, c, s, R, N, 0.0f, alpha, lr, q4, rope, glu, {}, {}, &dec))
+            return true;
+        gemm(prof_, 0, 1, T, N, K, A, K, w, K, C, N, dt, c, s, R, N, 0.0f, alpha, lr, q4, rope, glu);
+        return false;
+    };
+    // LoRA's xs = s x A^T of a projection stack (A [R, K])
+    auto lora_xs = [&](const void* in, const float* norm, int64_t R, int64_t K, int64_t a_off) {
+        if (ql) proj(in, norm, R, K, [&] { return W(a_off); }, xs.get(), dt, nullptr, lsc, nullptr, {}, {}, {}, {});
+    };
     hip::embed_fwd(ids, T, WB(emb_), V, d, xa.get(), dt, s);
     void* x = xa.get();
     void* xn = xb.get();
     for (int64_t l = 0; l < L; ++l) {
         const Layer& ly = layers_[l];
-        hip::rmsnorm_fwd(x, d, PB(ly.n1), h.get(), d, rr.as<float>(), T, d, eps, dt, s);
-        LowRank lq{};
-        if (ql) {
-            gemm(prof_, 0, 1, T, 3 * r, d, h.get(), d, W(ly.aqkv), d, xs.get(), 3 * r, dt, dt, s, nullptr, 0, 0.0f, lsc);
-            lq = LowRank{xs.get(), 3 * r, W(ly.bq), r, r, d, 0};
-        }
-        gemm(prof_, 0, 1, T, 3 * d, d, h.get(), d, wbase(ly, ly.wqkv, 0, 2), d, qkv.get(), 3 * d, dt, dt, s, nullptr,
-             0, 0.0f, 1.0f, ql ? &lq : nullptr, wq(ly, 0));
-        hip::rope(qkv.get(), 3 * d, B, S, 2 * H, hd, start_pos, cos_dev_, sin_dev_, false, dt, s);
-        // the new keys and values join the cache at rows start_pos .. start_pos + S - 1
+        // q, k (rotated) and v, the new keys and values also to the cache rows start_pos ..
+        // start_pos + S - 1
         char* kc = static_cast<char*>(kv_cache_) + es * static_cast<size_t>(l * 2 * B * MS * d);
         char* vc = kc + es * static_cast<size_t>(B * MS * d);
-        for (int64_t b = 0; b < B; ++b)
-            for (int kv = 0; kv < 2; ++kv)
-                AIC_HIP_CHECK(hipMemcpy2DAsync((kv ? vc : kc) + es * static_cast<size_t>((b * MS + start_pos) * d),
-                                               es * d, static_cast<char*>(qkv.get()) + es * ((b * S) * 3 * d + (1 + kv) * d),
-                                               es * 3 * d, es * d, S, hipMemcpyDeviceToDevice, s));
+        Decode cache;
+        cache.kc = kc;
+        cache.vc = vc;
+        cache.kv_rows = MS;
+        lora_xs(x, PB(ly.n1), 3 * r, d, ly.aqkv);
+        const LowRank lq{xs.get(), 3 * r, ql ? W(ly.bq) : nullptr, r, r, d, 0};
+        if (!proj(x, PB(ly.n1), 3 * d, d, [&] { return wbase(ly, ly.wqkv, 0, 2); }, qkv.get(), dt, nullptr, 1.0f,
+                  ql ? &lq : nullptr, wq(ly, 0), RopeOut{cos_dev_, sin_dev_, 2 * d, hd, S, start_pos}, {}, cache))
+            hip::kv_append(qkv.get(), kc, vc, B, S, d, MS, start_pos, dt, s);
         if (start_pos == 0)  // a fresh sequence: the flash kernel on the new rows is the same causal attention
             hip::attn_fwd(qkv.get(), static_cast<char*>(qkv.get()) + es * d, static_cast<char*>(qkv.get()) + es * 2 * d,
                           3 * d, ob.get(), d, lse.as<float>(), B, H, S, hd, true, scale, dt, s);
         else
             hip::attn_cached(qkv.get(), 3 * d, kc, vc, d, MS, ob.get(), d, B, H, S, start_pos, hd, scale, dt, s);
-        LowRank lo_{};
-        if (ql) {
-            gemm(prof_, 0, 1, T, r, d, ob.get(), d, W(ly.ao), d, xs.get(), r, dt, dt, s, nullptr, 0, 0.0f, lsc);
-            lo_ = LowRank{xs.get(), r, W(ly.bo), r, r, 0, 0};
-        }
-        gemm(prof_, 0, 1, T, d, d, ob.get(), d, wbase(ly, ly.wo, 3, 3), d, x1.get(), d, dt, dt, s, x, d, 0.0f, 1.0f,
-             ql ? &lo_ : nullptr, wq(ly, 3));
-        hip::rmsnorm_fwd(x1.get(), d, PB(ly.n2), h.get(), d, rr.as<float>(), T, d, eps, dt, s);
+        lora_xs(ob.get(), nullptr, r, d, ly.ao);
+        const LowRank lo_{xs.get(), r, ql ? W(ly.bo) : nullptr, r, r, 0, 0};
+        proj(ob.get(), nullptr, d, d, [&] { return wbase(ly, ly.wo, 3, 3); }, x1.get(), dt, x, 1.0f, ql ? &lo_ : nullptr,
+             wq(ly, 3), {}, {}, {});
         if (moe) {
+            hip::rmsnorm_fwd(x1.get(), d, PB(ly.n2), h.get(), d, rr.as<float>(), T, d, eps, dt, s);
             moe_[l]->forward(h.get(), T, W(ly.wr), W(ly.wex), x1.get(), xn, aux_dev_ + l, s);
         } else {
-            LowRank lg{};
-            if (ql) {
-                gemm(prof_, 0, 1, T, 2 * r, d, h.get(), d, W(ly.agu), d, xs.get(), 2 * r, dt, dt, s, nullptr, 0, 0.0f,
-                     lsc);
-                lg = LowRank{xs.get(), 2 * r, W(ly.bg), r, r, f, 0};
-            }
-            gemm(prof_, 0, 1, T, 2 * f, d, h.get(), d, wbase(ly, ly.wgu, 4, 5), d, gu.get(), 2 * f, dt, dt, s,
-                 nullptr, 0, 0.0f, 1.0f, ql ? &lg : nullptr, wq(ly, 4));
-            hip::swiglu_fwd(gu.get(), at(gu, f), 2 * f, am.get(), f, T, f, dt, s);
-            LowRank ld_{};
-            if (ql) {
-                gemm(prof_, 0, 1, T, r, f, am.get(), f, W(ly.ad), f, xs.get(), r, dt, dt, s, nullptr, 0, 0.0f, lsc);
-                ld_ = LowRank{xs.get(), r, W(ly.bd), r, r, 0, 0};
-            }
-            gemm(prof_, 0, 1, T, d, f, am.get(), f, wbase(ly, ly.wd, 6, 6), f, xn, d, dt, dt, s, x1.get(), d, 0.0f,
-                 1.0f, ql ? &ld_ : nullptr, wq(ly, 6));
+            Decode act_only;
+            act_only.skip_c = true;
+            lora_xs(x1.get(), PB(ly.n2), 2 * r, d, ly.agu);
+            const LowRank lg{xs.get(), 2 * r, ql ? W(ly.bg) : nullptr, r, r, f, 0};
+            proj(x1.get(), PB(ly.n2), 2 * f, d, [&] { return wbase(ly, ly.wgu, 4, 5); }, gu.get(), dt, nullptr, 1.0f,
+                 ql ? &lg : nullptr, wq(ly, 4), {}, GluOut{am.get(), f, f}, act_only);
+            lora_xs(am.get(), nullptr, r, f, ly.ad);
+            const LowRank ld_{xs.get(), r, ql ? W(ly.bd) : nullptr, r, r, 0, 0};
+            proj(am.get(), nullptr, d, f, [&] { return wbase(ly, ly.wd, 6, 6); }, xn, dt, x1.get(), 1.0f,
+                 ql ? &ld_ : nullptr, wq(ly, 6), {}, {}, {});
         }
         std::swap(x, xn);
     }
-    hip::rmsnorm_fwd(x, d, PB(normf_), h.get(), d, rr.as<float>(), T, d, eps, dt, s);
-    gemm(prof_, 0, 1, T, V, d, h.get(), d, WB(head_), d, logits, V, dt, DType::Float32, s);
+    proj(x, PB(normf_), V, d, [&] { return WB(head_); }, logits, DType::Float32, nullptr, 1.0f, nullptr, {}, {}, {}, {});
 }
 
 std::vector<int64_t> TransformerLM::generate(const std::vector<int64_t>& prompt, int64_t max_new_tokens,
