@@ -199,7 +199,8 @@ void launch_simt(const GemmArgs& a, hipStream_t s) {
 
 bool gemm_mfma_eligible(const GemmArgs& a) {
     if (a.ab != DType::BFloat16) return false;
-    if (a.K % 8 || a.lda % 8 || a.ldb % 8 || !aligned16(a.A) || !aligned16(a.B)) return false;
+    // K in 16-byte pieces where an operand is contiguous along it (a weight gradient's are not)
+    if (((!a.transA || a.transB) && a.K % 8) || a.lda % 8 || a.ldb % 8 || !aligned16(a.A) || !aligned16(a.B)) return false;
     if (a.transA && a.M % 8) return false;
     if (!a.transB && a.N % 8) return false;
     return true;
@@ -218,7 +219,7 @@ bool gemm_q4_eligible(const GemmArgs& a) {
 
 bool gemm_dma_eligible(const GemmArgs& a) {
     if (!gemm_mfma_eligible(a)) return false;
-    if (a.K % 64 || a.M < 8 || a.N < 8) return false;
+    if (((!a.transA || a.transB) && a.K % 64) || a.M < 8 || a.N < 8) return false;
     if (a.lda >= (int64_t{1} << 23) || a.ldb >= (int64_t{1} << 23)) return false;  // 32-bit copy offsets
     return true;
 }
@@ -473,7 +474,7 @@ void gemm(const GemmArgs& a, hipStream_t s) {
         int splits256 = 1;
         if (a.r2 == 0 && t256 < 256 && t256 >= 32 && a.K >= 4096) {
             splits256 = static_cast<int>(std::min<int64_t>(4, 256 / t256));
-            while (splits256 > 1 && a.K % (64LL * splits256)) --splits256;
+            while (splits256 > 1 && a.K / 64 % splits256) --splits256;
         }
         if (a.r2 > 0) {
             const int64_t bn = big ? 256 : 128;
@@ -496,7 +497,7 @@ void gemm(const GemmArgs& a, hipStream_t s) {
         int splits = 1;
         if (a.r2 == 0 && !big && t128 < 128 && a.K >= 1024) {
             splits = static_cast<int>(std::min<int64_t>({a.K / 512, (256 + t128 - 1) / t128, 16}));
-            while (splits > 1 && a.K % (64LL * splits)) --splits;
+            while (splits > 1 && a.K / 64 % splits) --splits;
         }
         if (splits > 1) {
             float* part = static_cast<float*>(stream_scratch(sizeof(float) * splits * a.M * a.N, s, 7));

@@ -19,7 +19,7 @@ constexpr int kDmaWaves256 = 8;
 // Register-staged MFMA kernel (shapes the DMA kernel cannot take).
 template <int BM, int BN, bool TA, bool TB, typename CT>
 void launch_mfma(const GemmArgs& a, hipStream_t s);
-// splits > 1: the K range is cut into `splits` equal parts (K % (64 splits) == 0), block z
+// splits > 1: the K range is cut into `splits` parts of equally many 64-deep tiles, block z
 // writes its fp32 partial to part + z M N (the caller reduces them).  Otherwise the low-rank
 // term of `a` (if any) runs in the kernel's tail.
 template <int BM, int BN, int BK, int S, bool TA, bool TB, typename CT>
