@@ -98,7 +98,7 @@ __global__ __launch_bounds__(256) void sq_matrix_k(const float* __restrict__ C, 
 }
 
 // ---------------------------------------------------------------------------------------
-// SIMT tiled GEMM (fp32 configuration, odd shapes).  64x64 tile, 256 threads, 4x4 each.
+// SIMT tiled GEMM (odd shapes).  64x64 tile, 256 threads, 4x4 each.
 // ---------------------------------------------------------------------------------------
 template <typename T, typename CT>
 __global__ __launch_bounds__(256) void gemm_simt(const T* __restrict__ A, const T* __restrict__ B, CT* C,
@@ -319,6 +319,17 @@ void gemm_q4(const GemmArgs& a, hipStream_t s) {
     }
 }
 
+void run_f32(const GemmArgs& a, hipStream_t s) {
+    const int parts = gemm_f32_parts(a);
+    if (parts == 1) {
+        gemm_f32(a, s);
+        return;
+    }
+    float* partial = static_cast<float*>(stream_scratch(sizeof(float) * parts * a.M * a.N, s, 7));
+    gemm_f32(a, s, parts, partial);
+    splitk_reduce(partial, parts, a, s);
+}
+
 // Few rows of x W^T: the kernel of gemm_skinny.hip (its low-rank term separately where the kernel
 // cannot take it).  False: not its shape.
 bool try_skinny(const GemmArgs& a, hipStream_t s) {
@@ -365,6 +376,10 @@ void gemm(const GemmArgs& a, hipStream_t s) {
                   InvalidArgument, "GEMM sums of squares: fp32 output only, without the RoPE / SwiGLU epilogues");
         // in the DMA tile kernels' epilogue or split-K reduction; the other paths (INT4 B, a
         // low-rank term, the non-DMA kernels) read the product back
+        if (gemm_f32_has_sq(a)) {
+            run_f32(a, s);
+            return;
+        }
         if (a.Bq || a.r2 > 0 || !gemm_dma_eligible(a)) {
             GemmArgs b = a;
             b.sq_part = nullptr;
@@ -542,9 +557,12 @@ void gemm(const GemmArgs& a, hipStream_t s) {
         }
         return;
     }
+    if (gemm_f32_eligible(a)) {
+        run_f32(a, s);
+        return;
+    }
     if (a.ab == DType::Float32) {
-        if (a.c == DType::Float32) launch_simt<float, float>(a, s);
-        else launch_simt<float, bf16>(a, s);
+        launch_simt<float, bf16>(a, s);
     } else {
         if (a.c == DType::Float32) launch_simt<bf16, float>(a, s);
         else launch_simt<bf16, bf16>(a, s);

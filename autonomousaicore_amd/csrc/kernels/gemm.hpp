@@ -110,6 +110,13 @@ struct SkinnyArgs {
 };
 bool gemm_skinny_eligible(const SkinnyArgs& q);
 void gemm_skinny(const SkinnyArgs& q, hipStream_t stream);
+// fp32 products of any shape and layout (gemm_f32.hip), in gemm_f32_parts(a) K parts: with more than
+// one, part z's sums go to partial + z M N and the caller adds them.  has_sq: the sums of squares
+// of `a` come out of its epilogue (its slots fit sq_cap) or out of that addition.
+bool gemm_f32_eligible(const GemmArgs& a);
+bool gemm_f32_has_sq(const GemmArgs& a);
+int gemm_f32_parts(const GemmArgs& a);
+void gemm_f32(const GemmArgs& a, hipStream_t stream, int parts = 1, float* partial = nullptr);
 // Independent products in one launch when they share the kernel configuration (transposes,
 // dtypes, alpha, beta; no residual or low-rank term; up to 8), so that their tiles fill the
 // chip together instead of each product's last partial round; otherwise one gemm() each.
