@@ -241,7 +241,7 @@ Plan plan_of(int64_t M, int64_t N, int64_t K) {
     q.tiles_m = (M + 16 * q.nt - 1) / (16 * q.nt);
     q.tiles_n = (N + 16 * q.nt - 1) / (16 * q.nt);
     q.split = 1;
-    while (q.split < kWaves && q.tiles_m * q.tiles_n * q.split < 2048 && K / 16 >= 8 * q.split) q.split *= 2;
+    while (q.split < kWaves && q.tiles_m * q.tiles_n * q.split < 2048 && K / 16 >= 2 * q.split) q.split *= 2;
     const int per = kWaves / q.split;
     q.blocks = static_cast<int>((q.tiles_m * q.tiles_n + per - 1) / per);
     return q;
