@@ -319,6 +319,12 @@ void gemm_q4(const GemmArgs& a, hipStream_t s) {
     }
 }
 
+// Rows that the fused RoPE / SwiGLU epilogues take: whole 256-row tiles, or any where the product
+// runs the persistent kernel (launch_dma), whose ragged form ends inside a tile.
+bool rows_fuse(const GemmArgs& a) {
+    return a.M % 256 == 0 || (!a.Bq && a.r2 == 0 && !a.transA && a.K % 128 == 0 && a.K >= 256);
+}
+
 void run_f32(const GemmArgs& a, hipStream_t s) {
     const int parts = gemm_f32_parts(a);
     if (parts == 1) {
@@ -399,8 +405,8 @@ void gemm(const GemmArgs& a, hipStream_t s) {
         // 128 (split in halves by the 64-column wave sub-tiles, exchanged through LDS) or 64 (one
         // per wave sub-tile), for the four-wave INT4 path heads of 128 (one per wave sub-tile,
         // after the kernel's low-rank term)
-        const bool tiles = a.c == DType::BFloat16 && a.M % 256 == 0 && a.N % 256 == 0 && a.rope_cols % 256 == 0 &&
-                           a.ldc % 8 == 0 && aligned16(a.C) && ((a.M / 256) * (a.N / 256) >= 128);
+        const bool tiles = a.c == DType::BFloat16 && rows_fuse(a) && a.N % 256 == 0 && a.rope_cols % 256 == 0 &&
+                           a.ldc % 8 == 0 && aligned16(a.C) && (((a.M + 255) / 256) * (a.N / 256) >= 128);
         const bool fused = tiles && (a.Bq ? a.rope_hd == 128 && a.transB && gemm_q4_eligible(a) &&
                                                 (a.r2 == 0 || rank_tail_ok(a, 256))
                                           : (a.rope_hd == 128 || a.rope_hd == 64) && gemm_impl::kDmaWaves256 == 8 &&
@@ -432,9 +438,9 @@ void gemm(const GemmArgs& a, hipStream_t s) {
         if (try_skinny(a, s)) return;
         // in the epilogue: bf16 x W^T on full 256x256 tiles of the eight-wave plain path, or of the
         // four-wave INT4 path (also after its low-rank term, whose segments follow the pairing)
-        const bool tiles = a.transB && !a.transA && a.c == DType::BFloat16 && a.M % 256 == 0 && a.glu_f % 128 == 0 &&
+        const bool tiles = a.transB && !a.transA && a.c == DType::BFloat16 && rows_fuse(a) && a.glu_f % 128 == 0 &&
                            a.ldc % 8 == 0 && aligned16(a.C) && a.ld_glu % 8 == 0 && aligned16(a.glu_out) &&
-                           ((a.M / 256) * (a.N / 256) >= 128);
+                           (((a.M + 255) / 256) * (a.N / 256) >= 128);
         const bool fused = tiles && (a.Bq ? gemm_q4_eligible(a) && (a.r2 == 0 || rank_tail_ok(a, 256))
                                           : gemm_impl::kDmaWaves256 == 8 && gemm_dma_eligible(a) && a.r2 == 0);
         if (!fused) {
@@ -456,8 +462,8 @@ void gemm(const GemmArgs& a, hipStream_t s) {
         // in the epilogue of the full-tile paths without K split (at least 128 tiles of 256x256)
         const int64_t es = static_cast<int64_t>(dtype_size(a.c));
         const bool fused = a.c == DType::BFloat16 && (a.Bq ? gemm_q4_eligible(a) : gemm_dma_eligible(a)) &&
-                           a.M % 256 == 0 && a.N % 256 == 0 &&
-                           (a.M / 256) * (a.N / 256) >= 128 && a.ldc % 8 == 0 && aligned16(a.C) &&
+                           rows_fuse(a) && a.N % 256 == 0 &&
+                           ((a.M + 255) / 256) * (a.N / 256) >= 128 && a.ldc % 8 == 0 && aligned16(a.C) &&
                            a.dglu_ld % 8 == 0 && aligned16(a.dglu_gu) && aligned16(a.dglu_out) &&
                            (a.r2 == 0 || rank_tail_ok(a, 256));  // C is not written: no rank term added later
         if (!fused) {
@@ -487,7 +493,8 @@ void gemm(const GemmArgs& a, hipStream_t s) {
         // under a round of 256x256 tiles over a long K (a 1024-wide head's input gradient: 128
         // tiles, K 32000): split K until about one round runs (682 -> 444 us there)
         int splits256 = 1;
-        if (a.r2 == 0 && t256 < 256 && t256 >= 32 && a.K >= 4096) {
+        const bool plain = a.r2 == 0 && !a.rope_cos && !a.dglu_gu;  // forms that the K splits' reduction has
+        if (plain && t256 < 256 && t256 >= 32 && a.K >= 4096) {
             splits256 = static_cast<int>(std::min<int64_t>(4, 256 / t256));
             while (splits256 > 1 && a.K / 64 % splits256) --splits256;
         }
@@ -510,7 +517,7 @@ void gemm(const GemmArgs& a, hipStream_t s) {
             return;
         }
         int splits = 1;
-        if (a.r2 == 0 && !big && t128 < 128 && a.K >= 1024) {
+        if (plain && !big && t128 < 128 && a.K >= 1024) {
             splits = static_cast<int>(std::min<int64_t>({a.K / 512, (256 + t128 - 1) / t128, 16}));
             while (splits > 1 && a.K / 64 % splits) --splits;
         }
@@ -525,7 +532,7 @@ void gemm(const GemmArgs& a, hipStream_t s) {
         // kernel beats a partial round of 256x256 tiles and two rounds of 128x128 ones (measured
         // 3-9% on those shapes); with a residual and at least half a round of 256x256 tiles the
         // persistent kernel stays ahead (its epilogue overlaps the next tile's copies)
-        if (a.r2 == 0 && !a.rope_cos && !a.dglu_gu && t256 < 256 && tw >= 128 && tw <= 256 && !(a.R && big)) {
+        if (plain && t256 < 256 && tw >= 128 && tw <= 256 && !(a.R && big)) {
             if (a.c == DType::Float32) dispatch_dma<128, 256, 64, 3, float>(a, s);
             else dispatch_dma<128, 256, 64, 3, bf16>(a, s);
             return;
