@@ -10,6 +10,7 @@
 #include <cstdint>
 
 #include "../runtime/dtype.hpp"
+#include "../kernels/kernels.hpp"
 #include "../runtime/memory_pool.hpp"
 
 namespace aic::models {
@@ -40,6 +41,8 @@ public:
     void backward(const void* dy, void* dx, float* dA, float* dB, bool accumulate, hipStream_t s);
 
 private:
+    bool one_pass(const hip::LoraSkinny& q) const;
+
     int64_t in_, out_, rank_, group_;
     float alpha_;
     DType scale_t_, dt_;
@@ -49,7 +52,7 @@ private:
     const void* B_ = nullptr;
     const uint8_t* Wq_ = nullptr;  // the frozen base, read again (dequantized) by backward
     const void* scales_ = nullptr;
-    DeviceBuffer xa_;
+    DeviceBuffer xs_;  // s x A^T of the forward
 };
 
 }  // namespace aic::models
