@@ -208,7 +208,7 @@ bool gemm_mfma_eligible(const GemmArgs& a) {
 
 bool gemm_q4_eligible(const GemmArgs& a) {
     if (!a.Bq || !a.Bscale || a.ab != DType::BFloat16 || a.transA) return false;
-    if (a.K <= 0 || a.K % 64 || a.M < 8 || a.N < 8 || a.lda % 8 || !aligned16(a.A) || !aligned16(a.Bq)) return false;
+    if (a.K <= 0 || a.K % 64 || a.M < 1 || a.N < 1 || a.lda % 8 || !aligned16(a.A) || !aligned16(a.Bq)) return false;
     if (a.scale_t != DType::Float16 || reinterpret_cast<uintptr_t>(a.Bscale) % 4) return false;
     if (a.group <= 0 || a.group % 64 || a.group >= (int64_t{1} << 31) || a.ldb % 64) return false;
     if (!a.transB && (a.N % 64 || a.ldb < a.N)) return false;
@@ -219,7 +219,8 @@ bool gemm_q4_eligible(const GemmArgs& a) {
 
 bool gemm_dma_eligible(const GemmArgs& a) {
     if (!gemm_mfma_eligible(a)) return false;
-    if (((!a.transA || a.transB) && a.K % 64) || a.M < 8 || a.N < 8) return false;
+    // (row copies clamp to the last row; a row-contiguous operand has at least 8 columns by then)
+    if (((!a.transA || a.transB) && a.K % 64) || a.M < 1 || a.N < 1) return false;
     if (a.lda >= (int64_t{1} << 23) || a.ldb >= (int64_t{1} << 23)) return false;  // 32-bit copy offsets
     return true;
 }
@@ -289,8 +290,9 @@ void rank_term_separately(const GemmArgs& a, hipStream_t s) {
 }  // namespace
 
 namespace {
-// The product with an INT4 B operand; tile size as for the bf16 operands (two stages on both),
-// never split along K.
+// The product with an INT4 B operand; tile size as for the bf16 operands (two stages on both), and
+// as there K split where few 128x128 tiles have a long one (5632 -> 2048 on 200 tokens, 32 tiles
+// over K 5632: 62 -> 20 us; 11264 -> 2048 on 64 114 -> 18).
 void gemm_q4(const GemmArgs& a, hipStream_t s) {
     AIC_CHECK(gemm_q4_eligible(a), InvalidArgument,
               "INT4 GEMM: unsupported shape or layout (bf16 A, K % 64, group % 64, ldb % 64, N % 64 for dy W)");
@@ -305,6 +307,21 @@ void gemm_q4(const GemmArgs& a, hipStream_t s) {
             rank_term_separately(a, s);
             return;
         }
+    }
+    const int64_t t128 = ((a.M + 127) / 128) * ((a.N + 127) / 128);
+    int splits = 1;
+    if (!big && t128 < 128 && a.K >= 1024) {
+        splits = static_cast<int>(std::min<int64_t>({a.K / 512, (256 + t128 - 1) / t128, 16}));
+        while (splits > 1 && a.K / 64 % splits) --splits;
+    } else if (!big && t128 <= 256 && a.K >= 4096 && a.K % 128 == 0) {
+        splits = 2;  // two of these blocks fit a CU
+    }
+    if (splits > 1) {
+        float* part = static_cast<float*>(stream_scratch(sizeof(float) * splits * a.M * a.N, s, 7));
+        a.transB ? gemm_impl::launch_dma_q4<128, 128, 64, 2, true, float>(a, s, splits, part)
+                 : gemm_impl::launch_dma_q4<128, 128, 64, 2, false, float>(a, s, splits, part);
+        splitk_reduce(part, splits, a, s);
+        return;
     }
     if (a.c == DType::Float32) {
         if (big) a.transB ? gemm_impl::launch_dma_q4<256, 256, 64, 2, true, float>(a, s)
@@ -343,7 +360,9 @@ bool try_skinny(const GemmArgs& a, hipStream_t s) {
     // again: a dense bf16 product stays on it only up to 4 M weights (64 rows: 2048x2048 11.5 us
     // against 14.2 on split tiles, 768x2048 11.4 against 14.7, 6144x2048 20.4 against 18.4, 32 rows:
     // 2048x5632 16.7 against 12.5, 11264x2048 18.7 against 15.8).
-    if (a.M > 16 && !a.Bq && a.ab == DType::BFloat16 && a.N * a.K > (int64_t{1} << 22)) return false;
+    // INT4 alike: 64 rows, 5632->2048 23 us against 14 on split tiles.
+    if (a.M > 16 && a.ab == DType::BFloat16 && a.N * a.K > (int64_t{1} << 22) && (!a.Bq || gemm_q4_eligible(a)))
+        return false;
     SkinnyArgs q;
     q.g = a;
     if (gemm_skinny_eligible(q)) {

@@ -86,7 +86,7 @@ struct GemmArgs {
 
 bool gemm_mfma_eligible(const GemmArgs& a);
 // The INT4 B operand in the kernel: bf16 A (not transposed, lda % 8, 16-byte aligned), K a
-// positive multiple of 64, M and N >= 8, fp16 scales (4-byte aligned base), group % 64 == 0,
+// positive multiple of 64, fp16 scales (4-byte aligned base), group % 64 == 0,
 // ldb % 64 == 0, Bq 16-byte aligned, N a multiple of 64 for the input-gradient layout, fewer
 // than 2^38 weight elements.
 bool gemm_q4_eligible(const GemmArgs& a);

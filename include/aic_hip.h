@@ -478,7 +478,7 @@ int aic_hip_int4_dequantize_zp(const uint8_t* packed, const float* scales, const
  * transW = 1: Wq holds W [N,K] and op(W) = W^T (forward y = x W^T); transW = 0: Wq holds W [K,N]
  * (input gradient dx = dy W).  With bf16 operands (ab_type AIC_BF16) in the shapes the GEMM
  * kernel takes (K % 64 == 0, group % 64 == 0, the weight's row length % 64 == 0, and for
- * transW = 0 N % 64 == 0; M, N >= 8; X and Wq 16-byte aligned) the packed values and scales are
+ * transW = 0 N % 64 == 0; X and Wq 16-byte aligned) the packed values and scales are
  * read by the GEMM itself and dequantized in its operand load, with no dequantized copy in HBM.
  * Otherwise (and for AIC_F32) the weight is first dequantized into library scratch in ab_type.
  * Either way op(W) holds q * scale rounded to ab_type, so both routes give the same product;
