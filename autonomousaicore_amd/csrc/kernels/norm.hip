@@ -122,23 +122,28 @@ __global__ __launch_bounds__(256) void rmsnorm_fwd_r(const T* __restrict__ x, in
     }
 }
 
-constexpr int kBwdRowsPerWave = 8;
+// Rows per wave of the backward: 8 (the next row's loads under this row's work, few partial rows)
+// as long as that leaves a block for every CU, fewer on fewer rows, where the chain of rows in a
+// wave is what the kernel takes.  bf16, both launches: 999 rows of 768, 32 blocks 15.2 us, one row
+// per wave 11.4 (7 of them the launches' own); 1000 of 2048, 23.1 -> 13.6; 4096 of 2048, 4 rows per
+// wave, 24.3 -> 19.6; 6000 of 2048, 6 rows, 25.7 -> 22.9; 8192 rows as before.
+int64_t bwd_rows_per_wave(int64_t rows) { return std::clamp<int64_t>((rows + 1023) / 1024, 1, 8); }
 
 // dx and per-block dw partials.  Block = 4 waves; wave w handles rows
-// blockIdx*16 + w*4 .. +3.  dw partial of the block -> part[blockIdx][dim].
+// (4 blockIdx + w) rpw .. + rpw - 1.  dw partial of the block -> part[blockIdx][dim].
 template <typename T, int VN>
 __global__ __launch_bounds__(256) void rmsnorm_bwd_k(const T* __restrict__ dy, int64_t lddy, const T* __restrict__ x,
                                                      int64_t ldx, const float* __restrict__ w,
                                                      const float* __restrict__ rms, const T* dres, int64_t ldres,
                                                      T* dx, int64_t lddx, float* __restrict__ part, int64_t rows,
-                                                     int dim) {
+                                                     int dim, int rpw) {
     extern __shared__ float sdw[];  // [4][dim] when part != nullptr
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     if (part)
         for (int j = threadIdx.x; j < 4 * dim; j += 256) sdw[j] = 0.0f;
     __syncthreads();
-    for (int rr = 0; rr < kBwdRowsPerWave; ++rr) {
-        const int64_t row = (static_cast<int64_t>(blockIdx.x) * 4 + wave) * kBwdRowsPerWave + rr;
+    for (int rr = 0; rr < rpw; ++rr) {
+        const int64_t row = (static_cast<int64_t>(blockIdx.x) * 4 + wave) * rpw + rr;
         if (row >= rows) break;
         const T* gr = dy + row * lddy;
         const T* xr = x + row * ldx;
@@ -181,19 +186,17 @@ __global__ __launch_bounds__(256) void rmsnorm_bwd_k(const T* __restrict__ dy, i
 }
 
 // Register-resident backward: wave w of block b handles rows (4b + w) R .. (4b + w) R + R - 1
-// (R = kBwdRegRowsPerWave, the loop form's count, so both write the same partial rows), with the
+// (R = rpw, as in the loop form, so both write the same partial rows), with the
 // next row's 16-byte chunks in flight while the current row is reduced and written (8 rows per
 // wave with this prefetch: 13% faster than 4 without it at the 1B shape, half the partial rows);
 // the lane's dw contributions accumulate in registers over its rows, then the four waves' sums
 // are added in wave order, as the loop form does through LDS.
-constexpr int kBwdRegRowsPerWave = 8;
-
 template <typename T, int VN, int CH>
 __global__ __launch_bounds__(256) void rmsnorm_bwd_r(const T* __restrict__ dy, int64_t lddy, const T* __restrict__ x,
                                                      int64_t ldx, const float* __restrict__ w,
                                                      const float* __restrict__ rms, const T* dres, int64_t ldres,
                                                      T* dx, int64_t lddx, float* __restrict__ part, int64_t rows,
-                                                     int dim) {
+                                                     int dim, int rpw) {
     extern __shared__ float sdw[];  // [4][dim] when part != nullptr
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     float wv[CH][VN], dwa[CH][VN];
@@ -236,9 +239,9 @@ __global__ __launch_bounds__(256) void rmsnorm_bwd_r(const T* __restrict__ dy, i
             }
         }
     };
-    const int64_t row0 = (static_cast<int64_t>(blockIdx.x) * 4 + wave) * kBwdRegRowsPerWave;
+    const int64_t row0 = (static_cast<int64_t>(blockIdx.x) * 4 + wave) * rpw;
     if (row0 < rows) fetch(row0);
-    for (int rr = 0; rr < kBwdRegRowsPerWave; ++rr) {
+    for (int rr = 0; rr < rpw; ++rr) {
         const int64_t row = row0 + rr;
         if (row >= rows) break;
         uint4 cg[CH], cx[CH], cr[CH];
@@ -249,7 +252,7 @@ __global__ __launch_bounds__(256) void rmsnorm_bwd_r(const T* __restrict__ dy, i
             cr[t] = nr[t];
         }
         const float r = nrm;
-        if (rr + 1 < kBwdRegRowsPerWave && row + 1 < rows) fetch(row + 1);
+        if (rr + 1 < rpw && row + 1 < rows) fetch(row + 1);
         float gv[CH][VN], xv[CH][VN];
 #pragma unroll
         for (int t = 0; t < CH; ++t) {
@@ -414,9 +417,8 @@ void bwd_t(const void* dy, int64_t lddy, const void* x, int64_t ldx, const float
     const bool vec = vec_ok(dy, lddy, dim, VN, sizeof(T)) && vec_ok(x, ldx, dim, VN, sizeof(T)) &&
                      vec_ok(dx, lddx, dim, VN, sizeof(T)) && (!dres || vec_ok(dres, ldres, dim, VN, sizeof(T)));
     const int ch = chunks_for(dim, VN);
-    const bool reg = vec && ch > 0;
-    const int64_t rows_per_block = 4 * (reg ? kBwdRegRowsPerWave : kBwdRowsPerWave);
-    const unsigned grid = static_cast<unsigned>((rows + rows_per_block - 1) / rows_per_block);
+    const int rpw = static_cast<int>(bwd_rows_per_wave(rows));
+    const unsigned grid = static_cast<unsigned>(rmsnorm_bwd_part_rows(rows));
     float* part = ext_part;  // the caller's partial rows (reduced later), or scratch reduced below
     if (dw && !part) part = static_cast<float*>(stream_scratch(sizeof(float) * grid * dim, s));
     const size_t lds = dw ? sizeof(float) * 4 * dim : 0;
@@ -424,7 +426,7 @@ void bwd_t(const void* dy, int64_t lddy, const void* x, int64_t ldx, const float
 #define AIC_BWD_R(CH)                                                                                         \
     hipLaunchKernelGGL((rmsnorm_bwd_r<T, VN, CH>), dim3(grid), dim3(256), lds, s, static_cast<const T*>(dy), \
                        lddy, static_cast<const T*>(x), ldx, w, rms, static_cast<const T*>(dres), ldres,        \
-                       static_cast<T*>(dx), lddx, part, rows, static_cast<int>(dim))
+                       static_cast<T*>(dx), lddx, part, rows, static_cast<int>(dim), rpw)
     if (vec && ch == 1) AIC_BWD_R(1);
     else if (vec && ch == 2) AIC_BWD_R(2);
     else if (vec && ch == 4) AIC_BWD_R(4);
@@ -433,11 +435,11 @@ void bwd_t(const void* dy, int64_t lddy, const void* x, int64_t ldx, const float
     else if (vec)
         hipLaunchKernelGGL((rmsnorm_bwd_k<T, VN>), dim3(grid), dim3(256), lds, s, static_cast<const T*>(dy), lddy,
                            static_cast<const T*>(x), ldx, w, rms, static_cast<const T*>(dres), ldres,
-                           static_cast<T*>(dx), lddx, part, rows, static_cast<int>(dim));
+                           static_cast<T*>(dx), lddx, part, rows, static_cast<int>(dim), rpw);
     else
         hipLaunchKernelGGL((rmsnorm_bwd_k<T, 1>), dim3(grid), dim3(256), lds, s, static_cast<const T*>(dy), lddy,
                            static_cast<const T*>(x), ldx, w, rms, static_cast<const T*>(dres), ldres,
-                           static_cast<T*>(dx), lddx, part, rows, static_cast<int>(dim));
+                           static_cast<T*>(dx), lddx, part, rows, static_cast<int>(dim), rpw);
     AIC_LAUNCH_CHECK("rmsnorm_bwd");
     if (dw && !ext_part) {
         if (dim % 8 == 0)
@@ -461,9 +463,10 @@ void rmsnorm_fwd(const void* x, int64_t ldx, const float* w, void* y, int64_t ld
     else AIC_THROW(DTypeMismatch, "rmsnorm_fwd: dtype must be f32 or bf16");
 }
 
-static_assert(kBwdRowsPerWave == kBwdRegRowsPerWave, "both backward forms take the same rows per block");
-
-int64_t rmsnorm_bwd_part_rows(int64_t rows) { return (rows + 4 * kBwdRowsPerWave - 1) / (4 * kBwdRowsPerWave); }
+int64_t rmsnorm_bwd_part_rows(int64_t rows) {
+    const int64_t per = 4 * bwd_rows_per_wave(rows);
+    return (rows + per - 1) / per;
+}
 
 void rmsnorm_bwd_deferred(const void* dy, int64_t lddy, const void* x, int64_t ldx, const float* w, const float* rms,
                           const void* dres, int64_t ldres, void* dx, int64_t lddx, float* part, int64_t rows,
