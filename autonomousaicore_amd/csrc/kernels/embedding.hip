@@ -1,8 +1,9 @@
 // Token embedding gather and its deterministic scatter-add backward.
 // Replaces cuda_embedding_forward/backward (src/cuda/cuda_embedding.cu:21-61), whose
 // backward uses fp32 atomicAdd (order-dependent results).  Here the backward sorts the
-// (id, position) pairs (chunks of 2048 sorted in LDS by as many blocks, then merged by rank:
-// each key's place is its index in its chunk plus its lower bound in every other chunk) and
+// (id, position) pairs (by counting up to 16384 tokens; beyond, chunks of 2048 sorted in LDS by as
+// many blocks, then merged by rank: each key's place is its index in its chunk plus its lower
+// bound in every other chunk) and
 // sums each id's rows in a fixed order (interleaved chains over the token-ordered run, then
 // the chains in order), so repeated runs are bit-identical and ids that repeat often
 // (Zipf-distributed text) are summed by sixteen waves instead of serialising on one address;
@@ -75,6 +76,50 @@ __global__ __launch_bounds__(1024) void embed_chunk_sort_k(const int64_t* __rest
         }
     }
     for (int i = threadIdx.x; i < n; i += blockDim.x) sk[c0 + i] = key[i];
+}
+
+// Up to this many tokens the sorted order comes from counting instead (embed_rank_k), and the runs
+// are found where they are summed.
+constexpr int64_t kRankTokens = 16384;
+constexpr int kRankBlock = 32;  // tokens ranked per block
+
+// The sorted order of N <= kRankTokens tokens by counting: token i's place is the number of tokens
+// with a smaller id plus the number of earlier ones with the same id.  Block b ranks tokens 32 b ..
+// 32 b + 31, one per lane of each half wave; the 32 half waves compare them with every 32nd four of
+// the ids, read from LDS as broadcasts, and add their counts.  N^2 compares, but with no barrier
+// between them, where the sort's passes are bound by theirs on one block per 2048 tokens and the
+// list of runs is one block's work.  The whole backward without the zeroing, bf16, 768 columns:
+// 64 tokens 35 -> 11 us, 999 37 -> 11, 8192 74 -> 24, 12000 81 -> 40, 16384 111 -> 48 (sort, merge
+// and list of runs before); 20000 tokens would already need 80 KB of LDS per block, which leaves
+// one block per CU, and keep the sort (119).
+__global__ __launch_bounds__(1024) void embed_rank_k(const int64_t* __restrict__ ids, int N, int64_t V,
+                                                     int* __restrict__ sorted_pos, int* __restrict__ sorted_id) {
+    extern __shared__ __attribute__((aligned(16))) unsigned rank_lds[];  // [quads][4]
+    __shared__ int part[32][kRankBlock];
+    const int quads = (N + kRankBlock - 1) / kRankBlock * (kRankBlock / 4);
+    const int lane = threadIdx.x & 31, slice = threadIdx.x >> 5;
+    for (int j = threadIdx.x; j < 4 * quads; j += 1024) {
+        const int64_t t = j < N ? ids[j] : -1;
+        rank_lds[j] = t >= 0 && t < V ? static_cast<unsigned>(t) : 0x7fffffffu;  // out of range: last
+    }
+    __syncthreads();
+    const int i = static_cast<int>(blockIdx.x) * kRankBlock + lane, own = static_cast<int>(blockIdx.x) * (kRankBlock / 4);
+    const unsigned my = rank_lds[i];
+    const uint4* q = reinterpret_cast<const uint4*>(rank_lds);
+    auto below = [](const uint4& v, unsigned t) { return (v.x < t) + (v.y < t) + (v.z < t) + (v.w < t); };
+    int count = 0, u = slice;
+#pragma unroll 4
+    for (; u < own; u += 32) count += below(q[u], my + 1);  // earlier tokens: equal ids count
+#pragma unroll 4
+    for (; u < quads; u += 32) count += below(q[u], my);
+    if (slice == 0)  // equal ids earlier in this block
+        for (int j = 0; j < lane; ++j) count += rank_lds[4 * own + j] == my;
+    part[slice][lane] = count;
+    __syncthreads();
+    if (slice != 0 || i >= N) return;
+    for (int w = 1; w < 32; ++w) count += part[w][lane];
+    sorted_pos[count] = i;
+    sorted_id[count] = static_cast<int>(my);
 }
 
 // The merged order: key g of chunk c lands at its index within c plus, for every other chunk,
@@ -232,49 +277,88 @@ __device__ __forceinline__ void sum_rows(float* acc, const int* __restrict__ sor
     }
 }
 
+// The end of the run of ids equal to id that starts at p, by all lanes of a wave: each round takes
+// the 64 equally spaced positions of the range that still holds it.
+__device__ __forceinline__ int run_end(const int* __restrict__ sorted_id, int N, int p, int id, int lane) {
+    int lo = p, span = N - p;  // lo is in the run, lo + span is not
+    while (span > 1) {
+        const int step = (span + 63) / 64, at = lo + lane * step;
+        const int hits = __popcll(__ballot(lane * step < span && sorted_id[at] == id));
+        const int next = lo + (hits - 1) * step;
+        span = min(step, lo + span - next);
+        lo = next;
+    }
+    return lo + 1;
+}
+
 // The column sums of every run of equal ids, per chunk of 64 lanes x LB bytes of the row.
 // Runs longer than kShortRun first: one block of 16 waves per (long run, chunk), wave w adding
 // the rows of tokens p + w, p + w + 16, ... in order, the 16 partial sums then added in wave
-// order.  Then the short runs: one wave per (run, chunk), adding the rows in token order.  Both
+// order.  Then the short runs: one wave per (run, chunk), adding the rows in token order.  The runs
+// come from the lists of embed_runs_k, or, where run_start is null, are found here, every sorted
+// position taken as the start of one and given up if it is not.  Both
 // orders are fixed by the run length alone, so the result is the same on every run.
 template <typename T, int LB>
 __global__ __launch_bounds__(1024) void embed_run_k(const int* __restrict__ sorted_pos, const int* __restrict__ sorted_id,
                                                     const int* __restrict__ run_start,
                                                     const int* __restrict__ long_runs, const int* __restrict__ counts,
-                                                    const T* __restrict__ dout, int64_t D, float* __restrict__ dW,
-                                                    int accumulate) {
+                                                    int N, const T* __restrict__ dout, int64_t D,
+                                                    float* __restrict__ dW, int accumulate) {
     constexpr int VE = LB / sizeof(T);  // elements per lane
     constexpr int CE = 64 * VE;         // columns per chunk
     __shared__ float part[16][CE];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int chunks = static_cast<int>(D / CE);
-    const int nruns = counts[0], nlong = counts[1];
-    for (int it = blockIdx.x; it < nlong * chunks; it += gridDim.x) {
-        const int r = long_runs[it / chunks], ch = it % chunks;
-        const int p = run_start[r], end = run_start[r + 1], id = sorted_id[p];
-        const int64_t col = static_cast<int64_t>(ch) * CE + lane * VE;
-        float acc[VE];
-#pragma unroll
-        for (int e = 0; e < VE; ++e) acc[e] = 0.0f;
-        sum_rows<T, LB, 8>(acc, sorted_pos, p + wave, end, 16, dout, D, col);
-#pragma unroll
-        for (int e = 0; e < VE; ++e) part[wave][lane * VE + e] = acc[e];
-        __syncthreads();
-        if (threadIdx.x < CE) {
-            float sum = part[0][threadIdx.x];
-#pragma unroll
-            for (int w = 1; w < 16; ++w) sum += part[w][threadIdx.x];
-            float* o = dW + static_cast<int64_t>(id) * D + static_cast<int64_t>(ch) * CE + threadIdx.x;
-            *o = accumulate ? *o + sum : sum;
+    const bool lists = run_start != nullptr;
+    const int nruns = lists ? counts[0] : N, nlong = lists ? counts[1] : N;
+    const int grid = static_cast<int>(gridDim.x), total = nlong * chunks;
+    for (int base = blockIdx.x; base < total; base += 64 * grid) {
+        // the block's next 64 items, one per lane; without lists only the starts of long runs count
+        bool want = lane < (total - base + grid - 1) / grid;
+        if (want && !lists) {
+            const int p = (base + lane * grid) / chunks, id = sorted_id[p];
+            want = id != 0x7fffffff && p + kShortRun < N && sorted_id[p + kShortRun] == id &&
+                   (p == 0 || sorted_id[p - 1] != id);
         }
-        __syncthreads();
+        for (unsigned long long todo = __ballot(want); todo; todo &= todo - 1) {
+            const int it = base + (__ffsll(todo) - 1) * grid, ch = it % chunks;
+            const int p = lists ? run_start[long_runs[it / chunks]] : it / chunks, id = sorted_id[p];
+            const int end = lists ? run_start[long_runs[it / chunks] + 1] : run_end(sorted_id, N, p, id, lane);
+            const int64_t col = static_cast<int64_t>(ch) * CE + lane * VE;
+            float acc[VE];
+#pragma unroll
+            for (int e = 0; e < VE; ++e) acc[e] = 0.0f;
+            sum_rows<T, LB, 8>(acc, sorted_pos, p + wave, end, 16, dout, D, col);
+#pragma unroll
+            for (int e = 0; e < VE; ++e) part[wave][lane * VE + e] = acc[e];
+            __syncthreads();
+            if (threadIdx.x < CE) {
+                float sum = part[0][threadIdx.x];
+#pragma unroll
+                for (int w = 1; w < 16; ++w) sum += part[w][threadIdx.x];
+                float* o = dW + static_cast<int64_t>(id) * D + static_cast<int64_t>(ch) * CE + threadIdx.x;
+                *o = accumulate ? *o + sum : sum;
+            }
+            __syncthreads();
+        }
     }
     const int gw = static_cast<int>(blockIdx.x) * 16 + wave, nw = static_cast<int>(gridDim.x) * 16;
     for (int it = gw; it < nruns * chunks; it += nw) {
         const int r = it / chunks, ch = it % chunks;
-        const int p = run_start[r], end = run_start[r + 1];
-        if (end - p > kShortRun) continue;
-        const int id = sorted_id[p];
+        int p, end, id;
+        if (lists) {
+            p = run_start[r], end = run_start[r + 1], id = sorted_id[p];
+            if (end - p > kShortRun) continue;
+        } else {
+            // lane l looks at position p - 1 + l; the run ends at the first other id after p
+            p = r;
+            const int at = p - 1 + lane, mine = at >= 0 && at < N ? sorted_id[at] : -1;
+            id = __shfl(mine, 1);
+            const unsigned long long same = __ballot(mine == id);
+            if (id == 0x7fffffff || (same & 1)) continue;
+            end = p + __ffsll(~(same >> 1)) - 1;
+            if (end - p > kShortRun) continue;
+        }
         const int64_t col = static_cast<int64_t>(ch) * CE + lane * VE;
         float acc[VE];
 #pragma unroll
@@ -374,27 +458,44 @@ void embed_bwd(const int64_t* ids, int64_t N, const void* dout, int64_t V, int64
     for (int b : {16, 8, 4})
         if (!lb && row_bytes % (64 * b) == 0 && (reinterpret_cast<uintptr_t>(dout) % b) == 0) lb = b;
     const bool runs = lb > 0 && vec;
-    auto* sk = static_cast<unsigned long long*>(stream_scratch(sizeof(unsigned long long) * N, s, 1));
     int* spos = static_cast<int*>(stream_scratch(sizeof(int) * (4 * N + 3), s));
     int* sid = spos + N;
     int* rstart = sid + N;      // N + 1 entries
     int* counts = rstart + N + 1;  // nruns, long runs
     int* lruns = counts + 2;
     const int n = static_cast<int>(N);
-    hipLaunchKernelGGL(embed_chunk_sort_k, dim3(static_cast<unsigned>((N + kSortChunk - 1) / kSortChunk)), dim3(1024),
-                       0, s, ids, n, V, sk);
-    AIC_LAUNCH_CHECK("embed_chunk_sort");
-    hipLaunchKernelGGL(embed_merge_rank_k, dim3(static_cast<unsigned>((N + 255) / 256)), dim3(256), 0, s, sk, n, spos,
-                       sid);
-    AIC_LAUNCH_CHECK("embed_merge_rank");
+    const bool by_rank = N <= kRankTokens;
+    if (by_rank) {
+        const unsigned blocks = static_cast<unsigned>((n + kRankBlock - 1) / kRankBlock);
+        static bool configured = false;
+        if (!configured) {
+            AIC_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(&embed_rank_k),
+                                              hipFuncAttributeMaxDynamicSharedMemorySize,
+                                              static_cast<int>(sizeof(unsigned) * kRankTokens)));
+            configured = true;
+        }
+        hipLaunchKernelGGL(embed_rank_k, dim3(blocks), dim3(1024), sizeof(unsigned) * kRankBlock * blocks, s, ids, n, V,
+                           spos, sid);
+        AIC_LAUNCH_CHECK("embed_rank");
+    } else {
+        auto* sk = static_cast<unsigned long long*>(stream_scratch(sizeof(unsigned long long) * N, s, 1));
+        hipLaunchKernelGGL(embed_chunk_sort_k, dim3(static_cast<unsigned>((N + kSortChunk - 1) / kSortChunk)),
+                           dim3(1024), 0, s, ids, n, V, sk);
+        AIC_LAUNCH_CHECK("embed_chunk_sort");
+        hipLaunchKernelGGL(embed_merge_rank_k, dim3(static_cast<unsigned>((N + 255) / 256)), dim3(256), 0, s, sk, n,
+                           spos, sid);
+        AIC_LAUNCH_CHECK("embed_merge_rank");
+    }
     if (!accumulate) {
         hipLaunchKernelGGL(embed_zero_absent_k, dim3(static_cast<unsigned>((V + 3) / 4)), dim3(256), 0, s, sid, n, V,
                            dW, D, vec);
         AIC_LAUNCH_CHECK("embed_zero_absent");
     }
     if (runs) {
-        hipLaunchKernelGGL(embed_runs_k, dim3(1), dim3(1024), 0, s, sid, n, V, rstart, lruns, counts);
-        AIC_LAUNCH_CHECK("embed_runs");
+        if (!by_rank) {
+            hipLaunchKernelGGL(embed_runs_k, dim3(1), dim3(1024), 0, s, sid, n, V, rstart, lruns, counts);
+            AIC_LAUNCH_CHECK("embed_runs");
+        }
         // a wave per (run, chunk) (16 per block), at most 2048 blocks striding
         const int64_t items = N * (row_bytes / (64 * lb));
         AIC_CHECK(items < (1LL << 31), InvalidArgument, "embed_bwd: tokens x row chunks exceeds 2^31");
@@ -402,8 +503,8 @@ void embed_bwd(const int64_t* ids, int64_t N, const void* dout, int64_t V, int64
         const int acc = accumulate ? 1 : 0;
         auto launch = [&](auto tag, auto lbc) {
             using T = decltype(tag);
-            hipLaunchKernelGGL((embed_run_k<T, decltype(lbc)::value>), dim3(g), dim3(1024), 0, s, spos, sid, rstart,
-                               lruns, counts, static_cast<const T*>(dout), D, dW, acc);
+            hipLaunchKernelGGL((embed_run_k<T, decltype(lbc)::value>), dim3(g), dim3(1024), 0, s, spos, sid,
+                               by_rank ? nullptr : rstart, lruns, counts, n, static_cast<const T*>(dout), D, dW, acc);
         };
         auto by_lb = [&](auto tag) {
             if (lb == 16) launch(tag, std::integral_constant<int, 16>{});
