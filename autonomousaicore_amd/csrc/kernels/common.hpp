@@ -153,6 +153,30 @@ inline unsigned grid_for(int64_t n, int block, int64_t cap = 65535LL * 8) {
     return static_cast<unsigned>(g);
 }
 
+// Map the hardware block id to a tile so that consecutive tiles (same A row panel,
+// neighbouring B panels) land on the same XCD.
+__device__ __forceinline__ int xcd_id(int bid, int nb) {
+    const int q = nb / 8, r = nb % 8;
+    const int xcd = bid % 8, local = bid / 8;
+    return (xcd < r) ? xcd * (q + 1) + local : r * (q + 1) + (xcd - r) * q + local;
+}
+
+// Tile of hardware block bid in groups of 4 row tiles: the 32 tiles an XCD runs at once span 4
+// A panels and 8 B panels (groups of 8, 16 and 32 rows measured 1.1%, 2.7% and 13% slower over
+// the 1B forward and input-gradient shapes; 1 or 4 rows with or without the XCD remap all within
+// 0.2%).
+__device__ __forceinline__ void tile_of(int bid, int nb, int tiles_m, int tiles_n, int& tm, int& tn) {
+    const int id = xcd_id(bid, nb);
+    constexpr int G = 4;
+    const int per_group = G * tiles_n;
+    const int group = id / per_group;
+    const int first_m = group * G;
+    const int gsize = min(tiles_m - first_m, G);
+    const int inner = id % per_group;
+    tm = first_m + inner % gsize;
+    tn = inner / gsize;
+}
+
 }  // namespace aic::hip
 
 #define AIC_LAUNCH_CHECK(what)                                                            \

@@ -54,35 +54,71 @@ __device__ __forceinline__ void sq_add1(double& acc, int& nf, float v) {
 
 // C = alpha * sum_z P[z] + beta * C + R over the split-K partials P [splits][M][N] (fp32,
 // summed in z order: deterministic); with sq, each block also writes the sum of squares of
-// the values it stored (one slot per block).
-template <typename CT>
+// the values it stored (one slot per block).  V elements of a row per thread: 4 (16-byte loads) where
+// rows and bases allow it, else 1.  Block (x, y) takes every gridDim.y-th stripe of 256 V elements of
+// the tile that the product's block x formed (tile x tile, in its order), so that where the tile
+// count is a multiple of 8 the partials are read on the XCD, from the L2, that wrote them:
+// 256x2048 in four parts of K 512, product and reduction, 12.3 us, 15.0 with 16-byte loads in row
+// order; 256x2304 14.0 (17.1 with 4-byte loads in row order), 1000x768 in four of 512 14.6 (17.4).
+template <typename CT, int V>
 __global__ __launch_bounds__(256) void splitk_reduce_k(const float* __restrict__ P, int splits, int64_t pz, int M, int N,
-                                                       float alpha, float beta, CT* C, int64_t ldc, const CT* R,
+                                                       int tile, float alpha, float beta, CT* C, int64_t ldc, const CT* R,
                                                        int64_t ldr, double* sq, int* sq_nf) {
-    const int64_t total = static_cast<int64_t>(M) * N;
+    struct alignas(4 * V) FV {
+        float v[V];
+    };
+    struct alignas(sizeof(CT) * V) CV {
+        CT v[V];
+    };
+    int tm, tn;
+    tile_of(blockIdx.x, gridDim.x, (M + tile - 1) / tile, (N + tile - 1) / tile, tm, tn);
+    const int rows = 256 * V / tile, n = tn * tile + static_cast<int>(threadIdx.x) * V % tile;
+    const int end = n < N ? min((tm + 1) * tile, M) : 0;
     double sqa = 0.0;
     int sqf = 0;
-    for (int64_t i = blockIdx.x * 256LL + threadIdx.x; i < total; i += static_cast<int64_t>(gridDim.x) * 256) {
-        const int m = static_cast<int>(i / N), n = static_cast<int>(i % N);
-        float acc = P[i];
+    for (int m = tm * tile + static_cast<int>(blockIdx.y) * rows + static_cast<int>(threadIdx.x) * V / tile; m < end;
+         m += rows * static_cast<int>(gridDim.y)) {
+        const int64_t i = static_cast<int64_t>(m) * N + n;
+        auto partial = [&](int z) { return *reinterpret_cast<const FV*>(P + z * pz + i); };
+        FV acc = partial(0);
+        auto add = [&](const FV& p) {
+#pragma unroll
+            for (int e = 0; e < V; ++e) acc.v[e] += p.v[e];
+        };
         int z = 1;
         // eight loads in flight, added in z order
         for (; z + 8 <= splits; z += 8) {
-            float p[8];
+            FV p[8];
 #pragma unroll
-            for (int u = 0; u < 8; ++u) p[u] = P[(z + u) * pz + i];
+            for (int u = 0; u < 8; ++u) p[u] = partial(z + u);
 #pragma unroll
-            for (int u = 0; u < 8; ++u) acc += p[u];
+            for (int u = 0; u < 8; ++u) add(p[u]);
         }
-        for (; z < splits; ++z) acc += P[z * pz + i];
-        const int64_t ci = static_cast<int64_t>(m) * ldc + n;
-        float v = alpha * acc;
-        if (beta != 0.0f) v += beta * ld(C, ci);
-        if (R) v += ld(R, static_cast<int64_t>(m) * ldr + n);
-        st(C, ci, v);
-        if (sq) sq_add1(sqa, sqf, v);  // fp32 C: the stored value
+        FV rest[7];
+#pragma unroll
+        for (int u = 0; u < 7; ++u)
+            if (z + u < splits) rest[u] = partial(z + u);
+#pragma unroll
+        for (int u = 0; u < 7; ++u)
+            if (z + u < splits) add(rest[u]);
+        CT* c = C + static_cast<int64_t>(m) * ldc + n;
+        CV old{}, res{}, out;
+        if (beta != 0.0f) old = *reinterpret_cast<const CV*>(c);
+        if (R) res = *reinterpret_cast<const CV*>(R + static_cast<int64_t>(m) * ldr + n);
+#pragma unroll
+        for (int e = 0; e < V; ++e) {
+            float v = alpha * acc.v[e];
+            if (beta != 0.0f) v += beta * ld(old.v, e);
+            if (R) v += ld(res.v, e);
+            st(out.v, e, v);
+            if (sq) sq_add1(sqa, sqf, v);  // fp32 C: the stored value
+        }
+        *reinterpret_cast<CV*>(c) = out;
     }
-    if (sq) sq_block256(sqa, sqf, sq + blockIdx.x, sq_nf + blockIdx.x);
+    if (sq) {
+        const unsigned slot = blockIdx.y * gridDim.x + blockIdx.x;
+        sq_block256(sqa, sqf, sq + slot, sq_nf + slot);
+    }
 }
 
 // Sums of squares of the fp32 matrix C [M, N] (leading dimension ldc), one slot per block: the
@@ -227,23 +263,57 @@ bool gemm_dma_eligible(const GemmArgs& a) {
 
 namespace {
 
-// C = alpha * (sum of the split-K partials) + beta * C + R (and the sums of squares of C when
-// a.sq_part is set: at most 1024 slots).
-void splitk_reduce(const float* part, int splits, const GemmArgs& a, hipStream_t s) {
-    const int64_t total = a.M * a.N;
-    const unsigned grid = static_cast<unsigned>(std::min<int64_t>((total + 255) / 256, a.sq_part ? 1024 : 4096));
+size_t partial_bytes(const GemmArgs& a, int parts) { return sizeof(float) * parts * a.M * a.N; }
+
+// C = alpha * (sum of the split-K partials) + beta * C + R, in the product's tile x tile tiles (and
+// the sums of squares of C when a.sq_part is set: at most 1024 slots).
+void splitk_reduce(const float* part, int splits, int tile, const GemmArgs& a, hipStream_t s) {
+    const int64_t total = a.M * a.N, es = static_cast<int64_t>(dtype_size(a.c));
+    const bool vec = a.N % 4 == 0 && a.ldc % 4 == 0 && reinterpret_cast<uintptr_t>(a.C) % (4 * es) == 0 &&
+                     (!a.R || (a.ldr % 4 == 0 && reinterpret_cast<uintptr_t>(a.R) % (4 * es) == 0)) &&
+                     reinterpret_cast<uintptr_t>(part) % 16 == 0;
+    const int64_t tiles = ((a.M + tile - 1) / tile) * ((a.N + tile - 1) / tile);
+    const int64_t stripes = int64_t{tile} * tile / (vec ? 1024 : 256);
+    const int64_t gy = std::max<int64_t>(1, std::min<int64_t>(stripes, (a.sq_part ? 1024 : 4096) / tiles));
+    const int64_t grid = tiles * gy;
+    AIC_CHECK(grid < (int64_t{1} << 31), InvalidArgument, "split-K reduction: too many tiles");
+    auto launch = [&](auto tag, auto v) {
+        using CT = decltype(tag);
+        hipLaunchKernelGGL((splitk_reduce_k<CT, decltype(v)::value>),
+                           dim3(static_cast<unsigned>(tiles), static_cast<unsigned>(gy)), dim3(256), 0, s, part, splits,
+                           total, static_cast<int>(a.M), static_cast<int>(a.N), tile, a.alpha, a.beta,
+                           static_cast<CT*>(a.C), a.ldc, static_cast<const CT*>(a.R), a.ldr, a.c == DType::Float32 ? a.sq_part : nullptr,
+                           a.c == DType::Float32 ? a.sq_nf : nullptr);
+    };
+    auto by_width = [&](auto tag) {
+        if (vec) launch(tag, std::integral_constant<int, 4>{});
+        else launch(tag, std::integral_constant<int, 1>{});
+    };
     if (a.c == DType::Float32) {
         AIC_CHECK(!a.sq_part || (a.sq_nf && grid <= a.sq_cap), InvalidArgument, "GEMM sums of squares: ", grid,
                   " slots needed, ", a.sq_cap, " given");
-        hipLaunchKernelGGL(splitk_reduce_k<float>, dim3(grid), dim3(256), 0, s, part, splits, total,
-                           static_cast<int>(a.M), static_cast<int>(a.N), a.alpha, a.beta, static_cast<float*>(a.C),
-                           a.ldc, static_cast<const float*>(a.R), a.ldr, a.sq_part, a.sq_nf);
+        by_width(float{});
     } else {
-        hipLaunchKernelGGL(splitk_reduce_k<bf16>, dim3(grid), dim3(256), 0, s, part, splits, total,
-                           static_cast<int>(a.M), static_cast<int>(a.N), a.alpha, a.beta, static_cast<bf16*>(a.C),
-                           a.ldc, static_cast<const bf16*>(a.R), a.ldr, nullptr, nullptr);
+        by_width(bf16{});
     }
     AIC_LAUNCH_CHECK("splitk_reduce_k");
+}
+
+// K parts of a product on 128x128 tiles of which one block fits a CU: few tiles over a long K fill
+// the chip with parts of it (the partials summed in a fixed order afterwards), at most one round of
+// blocks.  The part count with the least of: the chain along K, 6 ns a step of one column (measured
+// from K 768 to 8192), and, with parts, the reduction's launch and fill (4 us) and its traffic
+// (0.35 us per MB of partials).  2304x768 over K 1024 in one part 12.1 us (two parts, which any
+// product of fewer than 128 tiles was cut into, 18.4); 768x768 over K 8192 in four parts 22.6 (eight,
+// more than a round, 30.8; one 53.7); 1000x768 over K 3072 in four 16.4 (one 23.0).
+int dma_splits(int64_t t128, const GemmArgs& a) {
+    int best = 1;
+    double least = 6e-3 * a.K;
+    for (int n = 2; n <= std::min<int64_t>({a.K / 512, 256 / t128, 16}); ++n) {
+        const double t = 6e-3 * a.K / n + 4.0 + 1.4e-6 * n * a.M * a.N;
+        if (a.K / 64 % n == 0 && t < least) best = n, least = t;
+    }
+    return best;
 }
 
 // The sums of squares of the product already in C, for the paths without them in an epilogue.
@@ -316,11 +386,11 @@ void gemm_q4(const GemmArgs& a, hipStream_t s) {
     } else if (!big && t128 <= 256 && a.K >= 4096 && a.K % 128 == 0) {
         splits = 2;  // two of these blocks fit a CU
     }
-    if (splits > 1) {
-        float* part = static_cast<float*>(stream_scratch(sizeof(float) * splits * a.M * a.N, s, 7));
+    if (splits > 1 && stream_scratch_ready(partial_bytes(a, splits), s, 7)) {
+        float* part = static_cast<float*>(stream_scratch(partial_bytes(a, splits), s, 7));
         a.transB ? gemm_impl::launch_dma_q4<128, 128, 64, 2, true, float>(a, s, splits, part)
                  : gemm_impl::launch_dma_q4<128, 128, 64, 2, false, float>(a, s, splits, part);
-        splitk_reduce(part, splits, a, s);
+        splitk_reduce(part, splits, 128, a, s);
         return;
     }
     if (a.c == DType::Float32) {
@@ -344,13 +414,13 @@ bool rows_fuse(const GemmArgs& a) {
 
 void run_f32(const GemmArgs& a, hipStream_t s) {
     const int parts = gemm_f32_parts(a);
-    if (parts == 1) {
+    if (parts == 1 || !stream_scratch_ready(partial_bytes(a, parts), s, 7)) {
         gemm_f32(a, s);
         return;
     }
-    float* partial = static_cast<float*>(stream_scratch(sizeof(float) * parts * a.M * a.N, s, 7));
+    float* partial = static_cast<float*>(stream_scratch(partial_bytes(a, parts), s, 7));
     gemm_f32(a, s, parts, partial);
-    splitk_reduce(partial, parts, a, s);
+    splitk_reduce(partial, parts, 64, a, s);
 }
 
 // Few rows of x W^T: the kernel of gemm_skinny.hip (its low-rank term separately where the kernel
@@ -527,23 +597,17 @@ void gemm(const GemmArgs& a, hipStream_t s) {
                 return;
             }
         }
-        // few output tiles over a long K: split K so that the launch fills the chip (partials
-        // summed in a fixed order afterwards)
-        if (splits256 > 1) {
-            float* part = static_cast<float*>(stream_scratch(sizeof(float) * splits256 * a.M * a.N, s, 7));
+        if (splits256 > 1 && stream_scratch_ready(partial_bytes(a, splits256), s, 7)) {
+            float* part = static_cast<float*>(stream_scratch(partial_bytes(a, splits256), s, 7));
             dispatch_dma<256, 256, 64, 2, float>(a, s, splits256, part);
-            splitk_reduce(part, splits256, a, s);
+            splitk_reduce(part, splits256, 256, a, s);
             return;
         }
-        int splits = 1;
-        if (plain && !big && t128 < 128 && a.K >= 1024) {
-            splits = static_cast<int>(std::min<int64_t>({a.K / 512, (256 + t128 - 1) / t128, 16}));
-            while (splits > 1 && a.K / 64 % splits) --splits;
-        }
-        if (splits > 1) {
-            float* part = static_cast<float*>(stream_scratch(sizeof(float) * splits * a.M * a.N, s, 7));
+        const int splits = plain && !big ? dma_splits(t128, a) : 1;
+        if (splits > 1 && stream_scratch_ready(partial_bytes(a, splits), s, 7)) {
+            float* part = static_cast<float*>(stream_scratch(partial_bytes(a, splits), s, 7));
             dispatch_dma<128, 128, 64, 4, float>(a, s, splits, part);
-            splitk_reduce(part, splits, a, s);
+            splitk_reduce(part, splits, 128, a, s);
             return;
         }
         // under a round of 256x256 tiles where 128x256 tiles fill between half the chip and one

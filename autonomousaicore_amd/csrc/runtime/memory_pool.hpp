@@ -68,6 +68,11 @@ private:
 // bytes; callers use it only for the duration of their own launches.  Slots let one call hold
 // several buffers at once.
 void* stream_scratch(size_t bytes, hipStream_t stream, int slot = 0);
+// Whether stream_scratch gives `bytes` without an allocation inside a graph capture (an allocation
+// there would belong to the graph, and the kept pointer with it): what the stream has is large
+// enough, or the stream is not being captured.  A kernel form that needs scratch where another does
+// not is taken only then.
+bool stream_scratch_ready(size_t bytes, hipStream_t stream, int slot = 0);
 // Returns every scratch buffer cached for `stream` to the pool (stream-ordered on it); called
 // before the stream is destroyed, so that the buffers do not outlive it and a later stream at
 // the same handle address does not inherit them.
