@@ -21,13 +21,15 @@
 //
 // Where there are too few stationary tiles to fill the chip (decode, short chunks), `split`
 // waves of a block share one group of them, taking every split-th streaming block each, and add
-// their partial results through LDS in wave order: deterministic, no atomics, one launch.
+// their partial results through LDS in wave order: deterministic, no atomics, one launch.  A few
+// queries of a long cache are shared by blocks as well (key_parts), whose sums a second launch adds
+// in block order.
 //
 // Bound: short sequences by latency (a handful of dependent loads per wave), longer ones by the
 // MFMA pipe and LDS reads with 13 products where 7 are counted (the split probabilities).  Forward
 // and backward of 64 heads of 128, 128 queries on 2048 keys, bf16: 185 us (32.1 ms with the
 // one-thread-per-row kernels before); 512 queries 0.52 ms (74.8), fp32 1.83 ms (48.3); one query of
-// 12 heads of 64 on 2048 keys 43 us (6.1 ms).  Error against 64 bits as before in bf16 (1.7e-3, the
+// 12 heads of 64 on 2048 keys 10 us (6.1 ms).  Error against 64 bits as before in bf16 (1.7e-3, the
 // outputs' rounding) and 1.0e-6 (1.2e-6) in fp32.
 #include <algorithm>
 #include <cmath>
@@ -62,6 +64,8 @@ struct Args {
     int coff;       // key c is visible to query r when c <= r + coff
     int split;      // waves sharing a group of stationary rows (a divisor of the block's waves)
     int region;     // LDS bytes per wave
+    int parts;      // forward: blocks sharing one group of queries; > 1: attn_general_parts follows
+    float* part;    // their sums: [parts][B * H][Sq] rows of HD columns, then of m and l
     float scale;
 };
 
@@ -306,17 +310,37 @@ __device__ __forceinline__ void wait_lds() { asm volatile("s_waitcnt lgkmcnt(0)"
 
 extern __shared__ __attribute__((aligned(16))) char gen_lds[];
 
+// Query qi's output from exactly the keys it sees, one after the other.
+template <typename T, int HD>
+__device__ __forceinline__ void redo_row(const Args<T>& p, const T* qh, const T* kh, const T* vh, int64_t qi, T* out) {
+    const Row<T, HD> qr(qh + qi * p.ldq);
+    float mx = -INFINITY, sum = 0.0f, oa = 0.0f, ob = 0.0f;
+    for (int key = 0; key < min(p.Sk, static_cast<int>(qi) + p.coff + 1); ++key) {
+        const Row<T, HD> vr(vh + key * p.ldk);
+        const float x = qr.dot(Row<T, HD>(kh + key * p.ldk)) * p.scale, mn = fmaxf(mx, x);
+        const float f = exp_of<T>(mx - mn), e = exp_of<T>(x - mn);
+        sum = sum * f + e;
+        oa = oa * f + e * vr.a;
+        ob = ob * f + e * vr.b;
+        mx = mn;
+    }
+    store_row<T, HD>(out, oa / sum, ob / sum);
+}
+
 // ---------------------------------------------------------------------------------------
 // Forward: out0 = softmax(q k^T scale) v, lse.
 // ---------------------------------------------------------------------------------------
-template <typename T, int HD, int RT, bool VEC>
+// PARTS: block b / (B H) of a group takes every parts-th round of its keys and leaves its sums to
+// attn_general_parts.
+template <typename T, int HD, int RT, bool VEC, bool PARTS>
 __global__ __launch_bounds__(512) void attn_general_fwd(const Args<T> p) {
     using L = Lay<T, HD>;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, g = lane >> 4, c = lane & 15;
     const int nbh = p.B * p.H, bh = static_cast<int>(blockIdx.x) % nbh;
     const int per_block = (blockDim.x >> 6) / p.split;
     const int part = wave % p.split;
-    const int q0 = (static_cast<int>(blockIdx.x) / nbh * per_block + wave / p.split) * 16 * RT;
+    const int share = PARTS ? static_cast<int>(blockIdx.x) / nbh : 0;
+    const int q0 = PARTS ? 0 : (static_cast<int>(blockIdx.x) / nbh * per_block + wave / p.split) * 16 * RT;
     const int b = bh / p.H, h = bh % p.H;
     const T* qh = p.q + static_cast<int64_t>(b) * p.qb * p.ldq + static_cast<int64_t>(h) * HD;
     const T* kh = p.k + static_cast<int64_t>(b) * p.kb * p.ldk + static_cast<int64_t>(h) * HD;
@@ -350,8 +374,8 @@ __global__ __launch_bounds__(512) void attn_general_fwd(const Args<T> p) {
                 load_row<T, HD, VEC>(vh, row, p.ldk, vf[t]);
             }
         };
-        const int stride = kRows * p.split;
-        int k0 = kRows * part;
+        const int stride = kRows * p.split * (PARTS ? p.parts : 1);
+        int k0 = kRows * (share * p.split + part);
         if (k0 < kend) load(k0);
         for (; k0 < kend; k0 += stride) {
             wait_lds();  // the previous block's transposed reads
@@ -454,25 +478,26 @@ __global__ __launch_bounds__(512) void attn_general_fwd(const Args<T> p) {
 #pragma unroll
             for (int r = 0; r < RT; ++r) acc[dt][r] = *reinterpret_cast<const f32x4*>(region + ((dt * RT + r) * 64 + lane) * 16);
     }
+    if constexpr (PARTS) {
+        if (c >= p.Sq) return;
+        const int64_t row = (static_cast<int64_t>(share) * nbh + bh) * p.Sq + c;
+        float* st = p.part + static_cast<int64_t>(p.parts) * nbh * p.Sq * HD + 2 * row;
+        if (g == 0) {
+            st[0] = m[0];
+            st[1] = l[0];
+        }
+#pragma unroll
+        for (int dt = 0; dt < HD / 16; ++dt) *reinterpret_cast<f32x4*>(p.part + row * HD + 16 * dt + 4 * g) = acc[dt][0];
+        return;
+    }
 #pragma unroll
     for (int r = 0; r < RT; ++r) {
         const unsigned redo = non_finite<HD, RT>(acc, r);
         for (int u = 0; u < 16; ++u) {
             const int qi = q0 + 16 * r + u;
             if (!((redo >> u) & 1) || qi >= p.Sq) continue;
-            const Row<T, HD> qr(qh + qi * p.ldq);
-            float mx = -INFINITY, sum = 0.0f, oa = 0.0f, ob = 0.0f;
-            for (int key = 0; key < min(p.Sk, qi + p.coff + 1); ++key) {
-                const Row<T, HD> vr(vh + key * p.ldk);
-                const float x = qr.dot(Row<T, HD>(kh + key * p.ldk)) * p.scale, mn = fmaxf(mx, x);
-                const float f = exp_of<T>(mx - mn), e = exp_of<T>(x - mn);
-                sum = sum * f + e;
-                oa = oa * f + e * vr.a;
-                ob = ob * f + e * vr.b;
-                mx = mn;
-            }
-            store_row<T, HD>(p.out0 + (static_cast<int64_t>(b) * p.qb + qi) * p.ld0 + static_cast<int64_t>(h) * HD,
-                             oa / sum, ob / sum);
+            redo_row<T, HD>(p, qh, kh, vh, qi,
+                            p.out0 + (static_cast<int64_t>(b) * p.qb + qi) * p.ld0 + static_cast<int64_t>(h) * HD);
         }
         const int qi = q0 + 16 * r + c;
         if (qi >= p.Sq) continue;
@@ -484,6 +509,38 @@ __global__ __launch_bounds__(512) void attn_general_fwd(const Args<T> p) {
             const f32x4 a = acc[dt][r] / l[r];
             store4<VEC>(out + 16 * dt + 4 * g, a[0], a[1], a[2], a[3]);
         }
+    }
+}
+
+// The parts' sums of one query and head added in part order, one wave each.
+template <typename T, int HD>
+__global__ __launch_bounds__(64) void attn_general_parts(const Args<T> p) {
+    const int lane = threadIdx.x, nbh = p.B * p.H, rows = nbh * p.Sq, row = static_cast<int>(blockIdx.x);
+    const int bh = row / p.Sq, qi = row % p.Sq, b = bh / p.H, h = bh % p.H;
+    const float* st = p.part + static_cast<int64_t>(p.parts) * rows * HD;
+    const float m = lane < p.parts ? st[2 * (lane * static_cast<int64_t>(rows) + row)] : -INFINITY;
+    const float l = lane < p.parts ? st[2 * (lane * static_cast<int64_t>(rows) + row) + 1] : 0.0f;
+    float mx = m;
+#pragma unroll
+    for (int o = 1; o < 64; o *= 2) mx = fmaxf(mx, __shfl_xor(mx, o));
+    const float w = exp_of<T>(m - (mx == -INFINITY ? 0.0f : mx));
+    const float sum = wave_sum(w * l);
+    float oa = 0.0f, ob = 0.0f;
+#pragma unroll 4
+    for (int u = 0; u < p.parts; ++u) {
+        const Row<float, HD> v(p.part + (static_cast<int64_t>(u) * rows + row) * HD);
+        const float wu = __shfl(w, u);
+        oa = fmaf(wu, v.a, oa);
+        ob = fmaf(wu, v.b, ob);
+    }
+    T* out = p.out0 + (static_cast<int64_t>(b) * p.qb + qi) * p.ld0 + static_cast<int64_t>(h) * HD;
+    if (p.lse && lane == 0) p.lse[row] = mx + logf(sum);
+    if (__any(!(fabsf(oa) <= 3.402823466e38f) || !(fabsf(ob) <= 3.402823466e38f))) {  // as non_finite
+        const T* qh = p.q + static_cast<int64_t>(b) * p.qb * p.ldq + static_cast<int64_t>(h) * HD;
+        const int64_t kv = static_cast<int64_t>(b) * p.kb * p.ldk + static_cast<int64_t>(h) * HD;
+        redo_row<T, HD>(p, qh, p.k + kv, p.v + kv, qi, out);
+    } else {
+        store_row<T, HD>(out, oa / sum, ob / sum);
     }
 }
 
@@ -767,6 +824,17 @@ void choose(int64_t groups, int64_t blocks, int max_waves, int& waves, int& spli
     waves = std::max(4, split);
 }
 
+// Blocks sharing the keys of one group of up to 16 queries: one per round of 8 waves x 32 keys, as
+// far as the chip has a CU for each (16 x 12 heads, 2048 keys: two blocks each on fewer CUs 29 us,
+// one 24).  The second launch pays from 2816 bytes of a head's columns per streaming lane up, which
+// is 705 keys of 128 bytes or 353 of 256.  bf16, one query of 12 heads of 64: 768 keys 10.8 us in
+// one block and 9.8 in parts, 1001 12.1 and 10.0, 2048 19.2 and 10.2; 16 heads of 128: 257 keys
+// 10.2 and 11.2, 400 12.6 and 11.2, 2048 34.3 and 12.1; 4 x 16 heads, 2048 34.8 and 18.9.
+int key_parts(int64_t groups, int64_t blocks, int64_t row_bytes) {
+    if (blocks * row_bytes <= 2816) return 1;
+    return static_cast<int>(std::max<int64_t>(1, std::min<int64_t>({(blocks + 7) / 8, 256 / groups, 64})));
+}
+
 template <typename T, int HD, int RT, bool VEC, Kind K>
 void launch(Args<T> p, hipStream_t s) {
     constexpr int TILES = K == kDkDv ? 2 : 1;
@@ -779,21 +847,38 @@ void launch(Args<T> p, hipStream_t s) {
     int waves;
     choose(per * nbh, (stream + kRows - 1) / kRows, max_waves, waves, p.split);
     p.region = p.split > 1 ? REGION : ALONE;
-    const int64_t grid = (per + waves / p.split - 1) / (waves / p.split) * nbh;
+    int64_t grid = (per + waves / p.split - 1) / (waves / p.split) * nbh;
+    p.parts = 1;
+    if (K == kFwd && RT == 1 && per == 1 && p.split == max_waves) {
+        p.parts = key_parts(nbh, (std::min<int64_t>(p.Sk, p.Sq + static_cast<int64_t>(p.coff)) + kRows - 1) / kRows,
+                            static_cast<int64_t>(sizeof(T)) * HD);
+        const size_t bytes = sizeof(float) * p.parts * nbh * p.Sq * (HD + 2);
+        if (p.parts > 1 && !stream_scratch_ready(bytes, s)) p.parts = 1;
+        if (p.parts > 1) p.part = static_cast<float*>(stream_scratch(bytes, s));
+        grid *= p.parts;
+    }
     AIC_CHECK(grid < (int64_t{1} << 31), InvalidArgument, "attention: too many query or key blocks");
     void (*kernel)(Args<T>) = nullptr;
-    if constexpr (K == kFwd) kernel = attn_general_fwd<T, HD, RT, VEC>;
+    if constexpr (K == kFwd && RT == 1)
+        kernel = p.parts > 1 ? attn_general_fwd<T, HD, 1, VEC, true> : attn_general_fwd<T, HD, 1, VEC, false>;
+    else if constexpr (K == kFwd) kernel = attn_general_fwd<T, HD, RT, VEC, false>;
     else if constexpr (K == kDq) kernel = attn_general_dq<T, HD, RT, VEC>;
     else kernel = attn_general_dkdv<T, HD, RT, VEC>;
-    static bool configured = false;
-    if (!configured) {
+    static bool configured[2] = {};  // without and with parts
+    if (!configured[p.parts > 1]) {
         AIC_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
                                           hipFuncAttributeMaxDynamicSharedMemorySize, max_waves * REGION));
-        configured = true;
+        configured[p.parts > 1] = true;
     }
     hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(grid)), dim3(64 * waves),
                        static_cast<size_t>(waves) * p.region, s, p);
     AIC_LAUNCH_CHECK("attn_general");
+    if constexpr (K == kFwd && RT == 1) {
+        if (p.parts > 1) {
+            hipLaunchKernelGGL((attn_general_parts<T, HD>), dim3(static_cast<unsigned>(nbh * p.Sq)), dim3(64), 0, s, p);
+            AIC_LAUNCH_CHECK("attn_general_parts");
+        }
+    }
 }
 
 // Tiles of stationary rows per wave: two share every streaming fragment where the registers
