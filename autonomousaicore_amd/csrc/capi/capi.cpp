@@ -364,6 +364,7 @@ int aic_hip_gemm_swiglu_bwd(int64_t M, int64_t f, int64_t K, const void* A, int6
         a.dglu_gu = GU;
         a.dglu_out = DGU;
         a.dglu_ld = ldgu;
+        a.dglu_whole = true;  // the caller may read DH unless every tile is full
         aic::hip::gemm(a, st(stream));
     });
 }

@@ -8,7 +8,8 @@
 // This file holds the dispatch (tile shape, split-K, grouped and expert-ragged launches), the
 // split-K reduction and the SIMT kernel; the bf16 MFMA kernels are in gemm_kernels.inc,
 // instantiated per operand layout and output type by gemm_{nt,nn,tn,tt}_{bf16,f32}.hip.
-// fp32 path (the fp32 reference configuration) and odd shapes: a plain SIMT tiled kernel.
+// fp32 operands run gemm_f32.hip, up to 64 rows of x W^T gemm_skinny.hip; bf16 operands whose layout
+// the matrix kernels do not take, a plain SIMT tiled kernel.
 #include "gemm.hpp"
 
 #include <algorithm>
@@ -551,7 +552,7 @@ void gemm(const GemmArgs& a, hipStream_t s) {
         // in the epilogue of the full-tile paths without K split (at least 128 tiles of 256x256)
         const int64_t es = static_cast<int64_t>(dtype_size(a.c));
         const bool fused = a.c == DType::BFloat16 && (a.Bq ? gemm_q4_eligible(a) : gemm_dma_eligible(a)) &&
-                           rows_fuse(a) && a.N % 256 == 0 &&
+                           rows_fuse(a) && (a.M % 256 == 0 || !a.dglu_whole) && a.N % 256 == 0 &&
                            ((a.M + 255) / 256) * (a.N / 256) >= 128 && a.ldc % 8 == 0 && aligned16(a.C) &&
                            a.dglu_ld % 8 == 0 && aligned16(a.dglu_gu) && aligned16(a.dglu_out) &&
                            (a.r2 == 0 || rank_tail_ok(a, 256));  // C is not written: no rank term added later

@@ -67,12 +67,13 @@ struct GemmArgs {
     // Optional SwiGLU backward fed by the product (the down projection's input gradient
     // dh = dy W_d, [M, N = f]): with g = dglu_gu[row][j], u = dglu_gu[row][N + j] (leading
     // dimension dglu_ld) and dh the bf16 product, dglu_out[row][j] = dh u silu'(g) and
-    // dglu_out[row][N + j] = dh silu(g) (swiglu_bwd's arithmetic).  In the epilogue on full 256x256
+    // dglu_out[row][N + j] = dh silu(g) (swiglu_bwd's arithmetic).  In the epilogue on 256x256
     // tiles of bf16 output, where C is then not written; otherwise the product goes to C and
-    // swiglu_bwd runs after it.
+    // swiglu_bwd runs after it (with dglu_whole also where M ends inside a tile).
     const void* dglu_gu = nullptr;
     void* dglu_out = nullptr;
     int64_t dglu_ld = 0;
+    bool dglu_whole = false;
     // Optional sums of squares of the stored output (fp32 C only), for the gradient norm: the
     // call writes one fp64 partial and one non-finite flag per slot into sq_part[0..) /
     // sq_nf[0..) (at most sq_cap slots; how many depends on the path, always the same for the

@@ -73,3 +73,13 @@ def test_the_whole_product_is_right(ops):
     ref = ops["A"].double() @ ops["W"].double().T
     (C,) = run(ops, "plain", 300)
     assert float((C[:300].double() - ref[:300]).norm() / ref[:300].norm()) < 4e-3
+
+
+def test_swiglu_backward_keeps_the_product_of_a_partial_tile(ops):
+    M, p = 300, lambda t: t.data_ptr()  # noqa: E731
+    D, G, want = (torch.zeros((M, n), dtype=torch.bfloat16, device="cuda") for n in (N, 2 * N, N))
+    call("aic_hip_gemm_swiglu_bwd", M, N, K, p(ops["A"]), K, p(ops["Wt"]), N, p(ops["GU"]), 2 * N, p(D), N, p(G),
+         stream())
+    call("aic_hip_gemm", 0, 0, M, N, K, 1.0, p(ops["A"]), K, p(ops["Wt"]), N, 0.0, p(want), N, None, 0, BF16, BF16,
+         stream())
+    assert torch.equal(D, want)
