@@ -100,7 +100,8 @@ int aic_hip_gemm_lowrank(int transA, int transB, int64_t M, int64_t N, int64_t K
  * (bf16 A [M, K], W [N, K], C [M, N]) whose columns [0, rope_cols) are heads of hd values
  * rotated by the half-split RoPE at position start_pos + row % seq (cos_t / sin_t: [positions]
  * [hd / 2] tables as aic_hip_rope_tables builds them).  In the GEMM's epilogue for hd 128 on
- * shapes of at least 128 full 256 x 256 tiles; otherwise the product and then aic_hip_rope.
+ * shapes of at least 128 256 x 256 tiles (the last row tile may be partial); otherwise the product
+ * and then aic_hip_rope.
  * Replaces: Linear (q, k, v projections) followed by RotaryPositionEmbedding::forward on q and
  * k (include/nn/rope.hpp:23-112) as CausalSelfAttention::forward runs them. */
 int aic_hip_gemm_rope(int64_t M, int64_t N, int64_t K, const void* A, int64_t lda, const void* W, int64_t ldw,
@@ -109,8 +110,8 @@ int aic_hip_gemm_rope(int64_t M, int64_t N, int64_t K, const void* A, int64_t ld
 
 /* The FFN's gate/up projection with SwiGLU applied on the way out: GU = A W^T (bf16 A [M, K],
  * W [2f, K] = the gate rows then the up rows, GU [M, 2f]) and H[row][j] = silu(GU[row][j]) *
- * GU[row][f + j] (bf16 [M, f]).  In the GEMM's epilogue on shapes of at least 128 full 256 x 256
- * tiles with f % 128 == 0; otherwise the product and then aic_hip_swiglu_fwd.
+ * GU[row][f + j] (bf16 [M, f]).  In the GEMM's epilogue on shapes of at least 128 256 x 256 tiles (the
+ * last row tile may be partial) with f % 128 == 0; otherwise the product and then aic_hip_swiglu_fwd.
  * Replaces: the gate and up Linear layers followed by silu * mul (SwiGLU::forward,
  * include/nn/swiglu.hpp:21-33). */
 int aic_hip_gemm_swiglu(int64_t M, int64_t f, int64_t K, const void* A, int64_t lda, const void* W, int64_t ldw,
