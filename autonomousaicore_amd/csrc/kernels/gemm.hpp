@@ -109,6 +109,12 @@ struct SkinnyArgs {
     int64_t kv_rows = 0;
     bool skip_c = false;
 };
+// The segment of the low-rank term (seg_n) that the weight tile of rows row .. row + 15 takes.  A
+// block's second tile may lie past the last row, where no column is stored: the last row's segment,
+// so that X2 is read inside its rows.
+constexpr int low_rank_segment(int row, int N, int seg_n) {
+    return seg_n > 0 ? (row < N ? row : N - 1) / seg_n : 0;
+}
 bool gemm_skinny_eligible(const SkinnyArgs& q);
 void gemm_skinny(const SkinnyArgs& q, hipStream_t stream);
 // fp32 products of any shape and layout (gemm_f32.hip), in gemm_f32_parts(a) K parts: with more than

@@ -282,8 +282,7 @@ __global__ __launch_bounds__(64 * kWaves) void gemm_skinny_k(const SkinnyParams 
             Frag<D, 1, 1> fr;
 #pragma unroll
             for (int n = 0; n < NT; ++n) {
-                const int nt = n0 + n * p.pair;
-                const T* x2 = static_cast<const T*>(p.X2) + (p.seg_n > 0 ? nt / p.seg_n * p.r2 : 0);
+                const T* x2 = static_cast<const T*>(p.X2) + low_rank_segment(n0 + n * p.pair, p.N, p.seg_n) * p.r2;
                 fr.w[0] = ok ? *reinterpret_cast<const uint4*>(static_cast<const T*>(p.Y2) + wrow[n] * p.ldy2 + k)
                             : make_uint4(0, 0, 0, 0);
 #pragma unroll

@@ -68,6 +68,25 @@ def test_low_rank_term(ab, r2, M, seg):
     assert rel(host(out), ref) < TOL[ab]
 
 
+def test_low_rank_segments_past_the_last_tile():
+    """16464 columns in blocks of 32: the last block's second tile starts past the end, and its
+    low-rank columns with it.  X2 is the head of a larger buffer."""
+    rng = np.random.default_rng(9)
+    M, N, K, seg, r2 = 4, 16464, 64, 5488, 16
+    A, B, Y2, X2 = (mk(rng, BF16, *s) for s in ((M, K), (N, K), (N, r2), (M, r2 * N // seg)))
+    ref = A.astype(np.float64) @ B.astype(np.float64).T
+    for g in range(N // seg):
+        c = slice(g * seg, (g + 1) * seg)
+        ref[:, c] += X2[:, g * r2:(g + 1) * r2].astype(np.float64) @ Y2[c].astype(np.float64).T
+    a, b, y2 = (dev(x, T[BF16]) for x in (A, B, Y2))
+    buf = torch.full((X2.size + 1024,), float("nan"), dtype=T[BF16], device="cuda")
+    buf[:X2.size] = dev(X2, T[BF16]).reshape(-1)
+    out = torch.empty((M, N), dtype=T[BF16], device="cuda")
+    call("aic_hip_gemm_lowrank", 0, 1, M, N, K, 1.0, ptr(a), K, ptr(b), K, ptr(buf), X2.shape[1], ptr(y2), r2, r2, seg, 0, 0.0,
+         ptr(out), N, None, 0, BF16, BF16, stream())
+    assert rel(host(out), ref) < TOL[BF16]
+
+
 @pytest.mark.parametrize("B,S,H,hd,start", [(1, 1, 2, 64, 7), (3, 5, 4, 32, 0), (2, 32, 2, 128, 11)])
 def test_rotary_columns(B, S, H, hd, start):
     """The rotated q/k/v product equals the product followed by the rotary pass, to a bf16 unit."""
