@@ -853,7 +853,7 @@ void launch(Args<T> p, hipStream_t s) {
         p.parts = key_parts(nbh, (std::min<int64_t>(p.Sk, p.Sq + static_cast<int64_t>(p.coff)) + kRows - 1) / kRows,
                             static_cast<int64_t>(sizeof(T)) * HD);
         const size_t bytes = sizeof(float) * p.parts * nbh * p.Sq * (HD + 2);
-        if (p.parts > 1 && !stream_scratch_ready(bytes, s)) p.parts = 1;
+        if (p.parts > 1 && !stream_scratch_ready(s)) p.parts = 1;
         if (p.parts > 1) p.part = static_cast<float*>(stream_scratch(bytes, s));
         grid *= p.parts;
     }

@@ -387,7 +387,7 @@ void gemm_q4(const GemmArgs& a, hipStream_t s) {
     } else if (!big && t128 <= 256 && a.K >= 4096 && a.K % 128 == 0) {
         splits = 2;  // two of these blocks fit a CU
     }
-    if (splits > 1 && stream_scratch_ready(partial_bytes(a, splits), s, 7)) {
+    if (splits > 1 && stream_scratch_ready(s)) {
         float* part = static_cast<float*>(stream_scratch(partial_bytes(a, splits), s, 7));
         a.transB ? gemm_impl::launch_dma_q4<128, 128, 64, 2, true, float>(a, s, splits, part)
                  : gemm_impl::launch_dma_q4<128, 128, 64, 2, false, float>(a, s, splits, part);
@@ -415,7 +415,7 @@ bool rows_fuse(const GemmArgs& a) {
 
 void run_f32(const GemmArgs& a, hipStream_t s) {
     const int parts = gemm_f32_parts(a);
-    if (parts == 1 || !stream_scratch_ready(partial_bytes(a, parts), s, 7)) {
+    if (parts == 1 || !stream_scratch_ready(s)) {
         gemm_f32(a, s);
         return;
     }
@@ -598,14 +598,14 @@ void gemm(const GemmArgs& a, hipStream_t s) {
                 return;
             }
         }
-        if (splits256 > 1 && stream_scratch_ready(partial_bytes(a, splits256), s, 7)) {
+        if (splits256 > 1 && stream_scratch_ready(s)) {
             float* part = static_cast<float*>(stream_scratch(partial_bytes(a, splits256), s, 7));
             dispatch_dma<256, 256, 64, 2, float>(a, s, splits256, part);
             splitk_reduce(part, splits256, 256, a, s);
             return;
         }
         const int splits = plain && !big ? dma_splits(t128, a) : 1;
-        if (splits > 1 && stream_scratch_ready(partial_bytes(a, splits), s, 7)) {
+        if (splits > 1 && stream_scratch_ready(s)) {
             float* part = static_cast<float*>(stream_scratch(partial_bytes(a, splits), s, 7));
             dispatch_dma<128, 128, 64, 4, float>(a, s, splits, part);
             splitk_reduce(part, splits, 128, a, s);

@@ -115,15 +115,7 @@ void* stream_scratch(size_t bytes, hipStream_t stream, int slot) {
     return e.ptr;
 }
 
-bool stream_scratch_ready(size_t bytes, hipStream_t stream, int slot) {
-    {
-        int dev = 0;
-        AIC_HIP_CHECK(hipGetDevice(&dev));
-        std::lock_guard<std::mutex> lk(scratch_mu);
-        auto& cache = scratch_cache();
-        const auto it = cache.find(std::make_tuple(dev, stream, slot));
-        if (it != cache.end() && it->second.bytes >= bytes) return true;
-    }
+bool stream_scratch_ready(hipStream_t stream) {
     hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(stream, &status) != hipSuccess) {
         (void)hipGetLastError();  // the null stream beside another stream's capture

@@ -68,11 +68,10 @@ private:
 // bytes; callers use it only for the duration of their own launches.  Slots let one call hold
 // several buffers at once.
 void* stream_scratch(size_t bytes, hipStream_t stream, int slot = 0);
-// Whether stream_scratch gives `bytes` without an allocation inside a graph capture (an allocation
-// there would belong to the graph, and the kept pointer with it): what the stream has is large
-// enough, or the stream is not being captured.  A kernel form that needs scratch where another does
-// not is taken only then.
-bool stream_scratch_ready(size_t bytes, hipStream_t stream, int slot = 0);
+// Whether work on `stream` may use stream_scratch where another form does without: not while the
+// stream is captured.  A graph would keep the buffer's address, and the buffer goes back to the pool
+// when a later call needs a larger one or the stream's buffers are released.
+bool stream_scratch_ready(hipStream_t stream);
 // Returns every scratch buffer cached for `stream` to the pool (stream-ordered on it); called
 // before the stream is destroyed, so that the buffers do not outlive it and a later stream at
 // the same handle address does not inherit them.
