@@ -63,21 +63,23 @@ __device__ __forceinline__ void sq_add1(double& acc, int& nf, float v) {
 // order; 256x2304 14.0 (17.1 with 4-byte loads in row order), 1000x768 in four of 512 14.6 (17.4).
 template <typename CT, int V>
 __global__ __launch_bounds__(256) void splitk_reduce_k(const float* __restrict__ P, int splits, int64_t pz, int M, int N,
-                                                       int tile, float alpha, float beta, CT* C, int64_t ldc, const CT* R,
-                                                       int64_t ldr, double* sq, int* sq_nf) {
+                                                       int tile, int wshift, int tiles_m, int tiles_n, float alpha,
+                                                       float beta, CT* C, int64_t ldc, const CT* R, int64_t ldr,
+                                                       double* sq, int* sq_nf) {
     struct alignas(4 * V) FV {
         float v[V];
     };
     struct alignas(sizeof(CT) * V) CV {
         CT v[V];
     };
-    int tm, tn;
-    tile_of(blockIdx.x, gridDim.x, (M + tile - 1) / tile, (N + tile - 1) / tile, tm, tn);
-    const int rows = 256 * V / tile, n = tn * tile + static_cast<int>(threadIdx.x) * V % tile;
-    const int end = n < N ? min((tm + 1) * tile, M) : 0;
+    int tm = xcd_id(blockIdx.x, gridDim.x), tn = 0;
+    if (tiles_n > 1) tile_of(blockIdx.x, gridDim.x, tiles_m, tiles_n, tm, tn);
+    // stripes of 1 << wshift columns (divisions by a variable take 0.1 us each at this kernel's start)
+    const int rows = 256 * V >> wshift, at = static_cast<int>(threadIdx.x) * V;
+    const int n = tn * tile + (at & ((1 << wshift) - 1)), end = n < N ? min((tm + 1) * tile, M) : 0;
     double sqa = 0.0;
     int sqf = 0;
-    for (int m = tm * tile + static_cast<int>(blockIdx.y) * rows + static_cast<int>(threadIdx.x) * V / tile; m < end;
+    for (int m = tm * tile + static_cast<int>(blockIdx.y) * rows + (at >> wshift); m < end;
          m += rows * static_cast<int>(gridDim.y)) {
         const int64_t i = static_cast<int64_t>(m) * N + n;
         auto partial = [&](int z) { return *reinterpret_cast<const FV*>(P + z * pz + i); };
@@ -273,8 +275,10 @@ void splitk_reduce(const float* part, int splits, int tile, const GemmArgs& a, h
     const bool vec = a.N % 4 == 0 && a.ldc % 4 == 0 && reinterpret_cast<uintptr_t>(a.C) % (4 * es) == 0 &&
                      (!a.R || (a.ldr % 4 == 0 && reinterpret_cast<uintptr_t>(a.R) % (4 * es) == 0)) &&
                      reinterpret_cast<uintptr_t>(part) % 16 == 0;
-    const int64_t tiles = ((a.M + tile - 1) / tile) * ((a.N + tile - 1) / tile);
-    const int64_t stripes = int64_t{tile} * tile / (vec ? 1024 : 256);
+    const int64_t tm = (a.M + tile - 1) / tile, tn = (a.N + tile - 1) / tile, tiles = tm * tn;
+    int wshift = 2;  // columns of a stripe: the tile's, or where N ends early the power of two that holds them
+    while (1 << wshift < tile && int64_t{1} << wshift < a.N) ++wshift;
+    const int64_t stripes = std::max<int64_t>(1, (int64_t{tile} << wshift) / (vec ? 1024 : 256));
     const int64_t gy = std::max<int64_t>(1, std::min<int64_t>(stripes, (a.sq_part ? 1024 : 4096) / tiles));
     const int64_t grid = tiles * gy;
     AIC_CHECK(grid < (int64_t{1} << 31), InvalidArgument, "split-K reduction: too many tiles");
@@ -282,8 +286,9 @@ void splitk_reduce(const float* part, int splits, int tile, const GemmArgs& a, h
         using CT = decltype(tag);
         hipLaunchKernelGGL((splitk_reduce_k<CT, decltype(v)::value>),
                            dim3(static_cast<unsigned>(tiles), static_cast<unsigned>(gy)), dim3(256), 0, s, part, splits,
-                           total, static_cast<int>(a.M), static_cast<int>(a.N), tile, a.alpha, a.beta,
-                           static_cast<CT*>(a.C), a.ldc, static_cast<const CT*>(a.R), a.ldr, a.c == DType::Float32 ? a.sq_part : nullptr,
+                           total, static_cast<int>(a.M), static_cast<int>(a.N), tile, wshift, static_cast<int>(tm),
+                           static_cast<int>(tn), a.alpha, a.beta, static_cast<CT*>(a.C), a.ldc,
+                           static_cast<const CT*>(a.R), a.ldr, a.c == DType::Float32 ? a.sq_part : nullptr,
                            a.c == DType::Float32 ? a.sq_nf : nullptr);
     };
     auto by_width = [&](auto tag) {
@@ -307,13 +312,13 @@ void splitk_reduce(const float* part, int splits, int tile, const GemmArgs& a, h
 // (0.35 us per MB of partials).  2304x768 over K 1024 in one part 12.1 us (two parts, which any
 // product of fewer than 128 tiles was cut into, 18.4); 768x768 over K 8192 in four parts 22.6 (eight,
 // more than a round, 30.8; one 53.7); 1000x768 over K 3072 in four 16.4 (one 23.0).
+double dma_us(const GemmArgs& a, int parts) {
+    return 6e-3 * a.K / parts + (parts > 1 ? 4.0 + 1.4e-6 * parts * a.M * a.N : 0.0);
+}
 int dma_splits(int64_t t128, const GemmArgs& a) {
     int best = 1;
-    double least = 6e-3 * a.K;
-    for (int n = 2; n <= std::min<int64_t>({a.K / 512, 256 / t128, 16}); ++n) {
-        const double t = 6e-3 * a.K / n + 4.0 + 1.4e-6 * n * a.M * a.N;
-        if (a.K / 64 % n == 0 && t < least) best = n, least = t;
-    }
+    for (int n = 2; n <= std::min<int64_t>({a.K / 512, 256 / t128, 16}); ++n)
+        if (a.K / 64 % n == 0 && dma_us(a, n) < dma_us(a, best)) best = n;
     return best;
 }
 
@@ -434,6 +439,20 @@ bool try_skinny(const GemmArgs& a, hipStream_t s) {
     // INT4 alike: 64 rows, 5632->2048 23 us against 14 on split tiles.
     if (a.M > 16 && a.ab == DType::BFloat16 && a.N * a.K > (int64_t{1} << 22) && (!a.Bq || gemm_q4_eligible(a)))
         return false;
+    if (a.r2 == 0 && !a.Bq && gemm_dma_eligible(a)) {
+        // A block's eight waves walk all of K, 1 ns a column and 0.045 more for each row, so a long K is
+        // better cut among tile blocks, by more than the tiles' own fill and an epilogue's pass (64
+        // rows: 16 columns over K 5632 25 us here, 11 there; 16 over 32768 147 and 21; eight rows: 2048 over
+        // 5632 9.9 and 11.7, 256 over 8192 13.2 and 13.1, 64 over 16384 24.4 and 15.6).  Past 2^25 weights
+        // the tile copies read W faster (16 rows of 32000x2048: 26.9 us here, 21.1 there); not where
+        // their epilogue would round the bf16 product before it adds R or C.
+        const bool fused = a.rope_cos || a.glu_f > 0;
+        const int64_t t128 = (a.N + 127) / 128;
+        const int parts = stream_scratch_ready(s) ? dma_splits(t128, a) : 1;
+        if (a.K * (1e-3 + 4.5e-5 * a.M) > dma_us(a, parts) + (fused ? 6.5 : 2.5)) return false;
+        const bool adds = a.c == DType::BFloat16 && (a.R || a.beta != 0.0f);
+        if (!fused && !adds && a.N * a.K > (int64_t{1} << 25)) return false;
+    }
     SkinnyArgs q;
     q.g = a;
     if (gemm_skinny_eligible(q)) {

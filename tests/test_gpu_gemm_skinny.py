@@ -49,6 +49,50 @@ def test_product_with_alpha_beta_residual(ab, c, M, N, K):
         assert np.all(got[:, N:] == 9.0)
 
 
+def _small_ints(M, N, K):
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    return [torch.randint(-2, 3, s, generator=g, device="cuda").bfloat16() for s in ((M, K), (N, K), (M, N))]
+
+
+def _product(A, B, R, out):
+    (M, K), N = A.shape, B.shape[0]
+    call("aic_hip_gemm", 0, 1, M, N, K, 1.0, ptr(A), K, ptr(B), K, 0.0, ptr(out), N, ptr(R), N, BF16, BF16, stream())
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 16, 16384), (8, 16, 5632), (16, 16, 5632), (16, 24, 8192), (32, 40, 5632), (64, 264, 5632),
+                                   (64, 264, 2048), (1, 16400, 2048), (16, 16400, 2048), (64, 16, 33344), (64, 16, 5640)])
+def test_long_rows(M, N, K):
+    """Either side of the lengths and weight sizes from which a few-row product is cut among tile
+    blocks, a K that no part count divides and one outside the tiles' layouts.  The operands are
+    small integers: exact sums in any order, rounded once."""
+    A, B, R = _small_ints(M, N, K)
+    out, plain = torch.empty_like(R), torch.empty_like(R)
+    _product(A, B, R, out)
+    _product(A, B, None, plain)
+    ref = A.cpu().double() @ B.cpu().double().T
+    assert torch.equal(plain.cpu(), ref.to(torch.bfloat16))
+    assert torch.equal(out.cpu(), (ref + R.cpu().double()).to(torch.bfloat16))
+
+
+@pytest.mark.parametrize("N,K", [(16, 32768), (8, 65536), (256, 8192)])
+def test_few_long_rows_cost_no_more_than_more_rows(N, K):
+    """64 rows against 65, which never run the few-row kernel: 7 times the time there once."""
+    def us(M):
+        A, B, R = _small_ints(M, N, K)
+        out, a, b = torch.empty_like(R), torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        best = 1e9
+        for _ in range(6):
+            a.record()
+            for _ in range(30):
+                _product(A, B, R, out)
+            b.record()
+            torch.cuda.synchronize()
+            best = min(best, a.elapsed_time(b) * 1e3 / 30)
+        return best
+
+    assert us(64) < 2.0 * us(65)
+
+
 @pytest.mark.parametrize("M,seg", [(1, 0), (5, 96), (33, 32)])
 @pytest.mark.parametrize("r2", [8, 16, 40])
 @pytest.mark.parametrize("ab", [BF16, F32])
