@@ -27,7 +27,7 @@
 //
 // Bound: short sequences by latency (a handful of dependent loads per wave), longer ones by the
 // MFMA pipe and LDS reads with 13 products where 7 are counted (the split probabilities).  Forward
-// and backward of 64 heads of 128, 128 queries on 2048 keys, bf16: 185 us (32.1 ms with the
+// and backward of 64 heads of 128, 128 queries on 2048 keys, bf16: 172 us (32.1 ms with the
 // one-thread-per-row kernels before); 512 queries 0.52 ms (74.8), fp32 1.83 ms (48.3); one query of
 // 12 heads of 64 on 2048 keys 10 us (6.1 ms).  Error against 64 bits as before in bf16 (1.7e-3, the
 // outputs' rounding) and 1.0e-6 (1.2e-6) in fp32.
@@ -275,8 +275,11 @@ __device__ __forceinline__ void park(char* region, const f32x4 (&acc)[HD / 16][R
 
 // A hidden or missing row enters the tiles with weight zero, and zero times an infinity is NaN;
 // so is an infinity times the zero remainder of a bf16 weight.  Rows whose sums came out
-// non-finite are therefore computed again without tiles, one after the other, from exactly the
-// rows they see: bit c of the result is stationary row c of tile r.
+// non-finite are therefore summed again by `outer`, in fp32 and over exactly the rows they see: bit c
+// of the result is stationary row c of tile r.  Not where the row's weights are NaN themselves (a NaN or
+// an overflow in what it sees): then so is every sum.  64 heads of 64, 512 causal tokens, bf16,
+// forward and backward: 77 us, with NaN throughout 78, with an infinity in every value row 736 (15 ms each
+// when one wave formed such rows one after the other; 2.4 ms with one thread per row throughout).
 template <int HD, int RT>
 __device__ __forceinline__ unsigned non_finite(const f32x4 (&acc)[HD / 16][RT], int r) {
     bool bad = false;
@@ -287,44 +290,103 @@ __device__ __forceinline__ unsigned non_finite(const f32x4 (&acc)[HD / 16][RT], 
     const unsigned long long m = __ballot(bad);
     return static_cast<unsigned>((m | (m >> 16) | (m >> 32) | (m >> 48)) & 0xffffu);
 }
+// Bit c: x of stationary row c (every lane c of the four groups holds it) is a number.
+__device__ __forceinline__ unsigned numbers(float x) { return static_cast<unsigned>(__ballot(x == x) & 0xffffu); }
 
-// The row by row forms: a lane holds the head columns lane and lane + 64 of a row.
-template <typename T, int HD>
-struct Row {
-    float a, b;
-    __device__ __forceinline__ Row(const T* p) {
-        const int lane = threadIdx.x & 63;
-        a = lane < HD ? ld(p, lane) : 0.0f;
-        b = lane + 64 < HD ? ld(p, lane + 64) : 0.0f;
+__device__ __forceinline__ float vec_dot(const uint4& a, const uint4& b, float s) {
+    const uint32_t x[4] = {a.x, a.y, a.z, a.w}, y[4] = {b.x, b.y, b.z, b.w};
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        s = fmaf(__uint_as_float(x[e] << 16), __uint_as_float(y[e] << 16), s);
+        s = fmaf(__uint_as_float(x[e] & 0xffff0000u), __uint_as_float(y[e] & 0xffff0000u), s);
     }
-    __device__ __forceinline__ float dot(const Row& o) const { return wave_sum(fmaf(a, o.a, b * o.b)); }
-};
-template <typename T, int HD>
-__device__ __forceinline__ void store_row(T* p, float a, float b) {
-    const int lane = threadIdx.x & 63;
-    if (lane < HD) st(p, lane, a);
-    if (lane + 64 < HD) st(p, lane + 64, b);
+    return s;
 }
+__device__ __forceinline__ float vec_dot(const float4& a, const float4& b, float s) {
+    return fmaf(a.w, b.w, fmaf(a.z, b.z, fmaf(a.y, b.y, fmaf(a.x, b.x, s))));
+}
+
+// acc += X^T W as accumulate for one tile of stationary rows, a streaming row at a time and only
+// where seen(row) holds for this lane's stationary row; x: the weights as a lane holds them.
+__device__ __forceinline__ f32x4 four(const bf16* p) {
+    const uint2 u = *reinterpret_cast<const uint2*>(p);
+    return f32x4{__uint_as_float(u.x << 16), __uint_as_float(u.x & 0xffff0000u), __uint_as_float(u.y << 16),
+                 __uint_as_float(u.y & 0xffff0000u)};
+}
+__device__ __forceinline__ f32x4 four(const float* p) { return *reinterpret_cast<const f32x4*>(p); }
+template <typename T, int HD, typename Seen>
+__device__ __forceinline__ void outer(const char* tile, const float (&x)[2][4], Seen&& seen, f32x4 (&acc)[HD / 16]) {
+    const int lane = threadIdx.x & 63, g = lane >> 4, c = lane & 15;
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll 1
+            for (int j = 0; j < 4; ++j) {
+                const int row = 16 * t + 4 * j + i;
+                const T* p = reinterpret_cast<const T*>(tile + row * Lay<T, HD>::stride) + 4 * g;
+                const float w = __shfl(x[t][i], 16 * j + c);
+                if (seen(row)) {
+#pragma unroll
+                    for (int dt = 0; dt < HD / 16; ++dt) acc[dt] += w * four(p + 16 * dt);
+                }
+            }
+}
+
+// The same for one query (attn_general_parts): 64 keys at a time, a lane each for the products of whole rows
+// (row_dot), then the lanes as columns for the weighted sums (Sums): lane l holds the columns l % 64
+// and l % 64 + 64 of a head, heads of 16 and 32 in groups of lanes with every 4th and 2nd row.
+template <typename T, int HD>
+__device__ __forceinline__ float row_dot(const T* a, const T* b) {
+    float s = 0.0f;
+#pragma unroll 4
+    for (int c = 0; c < HD; c += Lay<T, HD>::width) s = vec_dot(load_vec<false>(a + c), load_vec<false>(b + c), s);
+    return s;
+}
+template <typename T, int HD>
+struct Sums {
+    static constexpr int C = HD < 64 ? HD : 64, G = 64 / C;
+    float a = 0.0f, b = 0.0f;
+    // += the rows p, p + ld, ... of n lanes, weighted by each lane's w
+    __device__ __forceinline__ void add(const T* p, int64_t ld, int n, float w) {
+        const int lane = threadIdx.x & 63, g = lane / C, c = lane % C;
+#pragma unroll 8
+        for (int j = 0; j < n; j += G) {
+            const int r = min(j + g, n - 1);
+            const float x = aic::hip::ld(p + r * ld, c), y = HD > 64 ? aic::hip::ld(p + r * ld, c + 64) : 0.0f;
+            const float wr = __shfl(w, r);
+            if (j + g < n) {
+                a = fmaf(wr, x, a);
+                if (HD > 64) b = fmaf(wr, y, b);
+            }
+        }
+    }
+    __device__ __forceinline__ void store(T* p, float f) {
+        const int lane = threadIdx.x & 63;
+#pragma unroll
+        for (int o = C; o < 64; o *= 2) a += __shfl_xor(a, o);
+        if (lane < HD) st(p, lane, a * f);
+        if (HD > 64) st(p, lane + 64, b * f);
+    }
+};
 
 __device__ __forceinline__ void wait_lds() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
 
 extern __shared__ __attribute__((aligned(16))) char gen_lds[];
 
-// Query qi's output from exactly the keys it sees, one after the other.
+// Query qi's output from exactly the keys it sees; m and l: its scores' maximum and weights' sum.
 template <typename T, int HD>
-__device__ __forceinline__ void redo_row(const Args<T>& p, const T* qh, const T* kh, const T* vh, int64_t qi, T* out) {
-    const Row<T, HD> qr(qh + qi * p.ldq);
-    float mx = -INFINITY, sum = 0.0f, oa = 0.0f, ob = 0.0f;
-    for (int key = 0; key < min(p.Sk, static_cast<int>(qi) + p.coff + 1); ++key) {
-        const Row<T, HD> vr(vh + key * p.ldk);
-        const float x = qr.dot(Row<T, HD>(kh + key * p.ldk)) * p.scale, mn = fmaxf(mx, x);
-        const float f = exp_of<T>(mx - mn), e = exp_of<T>(x - mn);
-        sum = sum * f + e;
-        oa = oa * f + e * vr.a;
-        ob = ob * f + e * vr.b;
-        mx = mn;
+__device__ __forceinline__ void redo_row(const Args<T>& p, const T* qh, const T* kh, const T* vh, int64_t qi, float m,
+                                         float l, T* out) {
+    const int lane = threadIdx.x & 63, end = min(p.Sk, static_cast<int>(qi) + p.coff + 1);
+    const float base = m == -INFINITY ? 0.0f : m;
+    Sums<T, HD> o;
+    for (int k0 = 0; k0 < end; k0 += 64) {
+        const int n = min(64, end - k0);
+        const float x = row_dot<T, HD>(qh + qi * p.ldq, kh + (k0 + min(lane, n - 1)) * p.ldk) * p.scale;
+        o.add(vh + k0 * p.ldk, p.ldk, n, exp_of<T>(x - base));
     }
-    store_row<T, HD>(out, oa / sum, ob / sum);
+    o.store(out, 1.0f / l);
 }
 
 // ---------------------------------------------------------------------------------------
@@ -490,24 +552,53 @@ __global__ __launch_bounds__(512) void attn_general_fwd(const Args<T> p) {
         for (int dt = 0; dt < HD / 16; ++dt) *reinterpret_cast<f32x4*>(p.part + row * HD + 16 * dt + 4 * g) = acc[dt][0];
         return;
     }
+    unsigned redo = 0;  // bit 16 r + c: row c of tile r
+    T* out = p.out0 + (static_cast<int64_t>(b) * p.qb + q0 + c) * p.ld0 + static_cast<int64_t>(h) * HD + 4 * g;
 #pragma unroll
     for (int r = 0; r < RT; ++r) {
-        const unsigned redo = non_finite<HD, RT>(acc, r);
-        for (int u = 0; u < 16; ++u) {
-            const int qi = q0 + 16 * r + u;
-            if (!((redo >> u) & 1) || qi >= p.Sq) continue;
-            redo_row<T, HD>(p, qh, kh, vh, qi,
-                            p.out0 + (static_cast<int64_t>(b) * p.qb + qi) * p.ld0 + static_cast<int64_t>(h) * HD);
-        }
+        const unsigned bad = non_finite<HD, RT>(acc, r) & numbers(l[r]);
+        redo |= bad << (16 * r);
         const int qi = q0 + 16 * r + c;
         if (qi >= p.Sq) continue;
         if (p.lse && g == 0) p.lse[(static_cast<int64_t>(b) * p.H + h) * p.Sq + qi] = m[r] + logf(l[r]);
-        if ((redo >> c) & 1) continue;
-        T* out = p.out0 + (static_cast<int64_t>(b) * p.qb + qi) * p.ld0 + static_cast<int64_t>(h) * HD;
+        if ((bad >> c) & 1) continue;
 #pragma unroll
         for (int dt = 0; dt < HD / 16; ++dt) {
             const f32x4 a = acc[dt][r] / l[r];
-            store4<VEC>(out + 16 * dt + 4 * g, a[0], a[1], a[2], a[3]);
+            store4<VEC>(out + 16 * r * p.ld0 + 16 * dt, a[0], a[1], a[2], a[3]);
+        }
+    }
+#pragma unroll 1
+    for (int r = 0; r < RT; ++r) {
+        if (!((redo >> (16 * r)) & 0xffffu)) continue;
+        const int qi = q0 + 16 * r + c, end = min(p.Sk, qi + p.coff + 1);
+        const int kend = min(p.Sk, min(q0 + 16 * r + 16, p.Sq) + p.coff);
+        const float mr = RT > 1 && r ? m[RT - 1] : m[0], lr = RT > 1 && r ? l[RT - 1] : l[0];
+        const float base = mr == -INFINITY ? 0.0f : mr;
+        typename L::Vec qf[L::frags], f[L::frags];
+        load_row<T, HD, VEC>(qh, min(qi, p.Sq - 1), p.ldq, qf);
+        f32x4 sum[HD / 16] = {};
+        for (int k0 = 0; k0 < kend; k0 += kRows) {
+            float x[2][4];
+            wait_lds();
+#pragma unroll
+            for (int t = 0; t < 2; ++t) {
+                const int row = min(k0 + 16 * t + c, p.Sk - 1);
+                load_row<T, HD, VEC>(vh, row, p.ldk, f);
+                store_lds<T, HD>(region, 16 * t + c, f);
+                load_row<T, HD, VEC>(kh, row, p.ldk, f);
+                const f32x4 s = dot<HD>(f, qf);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) x[t][i] = exp_of<T>(s[i] * p.scale - base);
+            }
+            wait_lds();
+            outer<T, HD>(region, x, [&](int row) { return k0 + row < end; }, sum);
+        }
+        if (qi >= p.Sq || !((redo >> (16 * r + c)) & 1)) continue;
+#pragma unroll
+        for (int dt = 0; dt < HD / 16; ++dt) {
+            const f32x4 a = sum[dt] / lr;
+            store4<VEC>(out + 16 * r * p.ld0 + 16 * dt, a[0], a[1], a[2], a[3]);
         }
     }
 }
@@ -528,19 +619,21 @@ __global__ __launch_bounds__(64) void attn_general_parts(const Args<T> p) {
     float oa = 0.0f, ob = 0.0f;
 #pragma unroll 4
     for (int u = 0; u < p.parts; ++u) {
-        const Row<float, HD> v(p.part + (static_cast<int64_t>(u) * rows + row) * HD);
+        const float* v = p.part + (static_cast<int64_t>(u) * rows + row) * HD;
         const float wu = __shfl(w, u);
-        oa = fmaf(wu, v.a, oa);
-        ob = fmaf(wu, v.b, ob);
+        oa = fmaf(wu, lane < HD ? v[lane] : 0.0f, oa);
+        ob = fmaf(wu, lane + 64 < HD ? v[lane + 64] : 0.0f, ob);
     }
     T* out = p.out0 + (static_cast<int64_t>(b) * p.qb + qi) * p.ld0 + static_cast<int64_t>(h) * HD;
     if (p.lse && lane == 0) p.lse[row] = mx + logf(sum);
-    if (__any(!(fabsf(oa) <= 3.402823466e38f) || !(fabsf(ob) <= 3.402823466e38f))) {  // as non_finite
+    const bool bad = !(fabsf(oa) <= 3.402823466e38f) || !(fabsf(ob) <= 3.402823466e38f);
+    if (sum == sum && __any(bad)) {  // as non_finite
         const T* qh = p.q + static_cast<int64_t>(b) * p.qb * p.ldq + static_cast<int64_t>(h) * HD;
         const int64_t kv = static_cast<int64_t>(b) * p.kb * p.ldk + static_cast<int64_t>(h) * HD;
-        redo_row<T, HD>(p, qh, p.k + kv, p.v + kv, qi, out);
+        redo_row<T, HD>(p, qh, p.k + kv, p.v + kv, qi, mx, sum, out);
     } else {
-        store_row<T, HD>(out, oa / sum, ob / sum);
+        if (lane < HD) aic::hip::st(out, lane, oa / sum);
+        if (lane + 64 < HD) aic::hip::st(out, lane + 64, ob / sum);
     }
 }
 
@@ -574,10 +667,10 @@ __global__ __launch_bounds__(256) void attn_general_dq(const Args<T> p) {
     char* region = gen_lds + wave * p.region;
 
     f32x4 acc[HD / 16][RT] = {};
+    float lse[RT] = {}, D[RT] = {};
     if (q0 < p.Sq) {
         typename L::Vec qf[RT][L::frags], df[RT][L::frags];
         int vis[RT];
-        float lse[RT], D[RT];
 #pragma unroll
         for (int r = 0; r < RT; ++r) {
             const int qi = min(q0 + 16 * r + c, p.Sq - 1);
@@ -590,21 +683,7 @@ __global__ __launch_bounds__(256) void attn_general_dq(const Args<T> p) {
             load_row<T, HD, VEC>(p.o + tok0 * p.ldo + hoff, qi, p.ldo, of);
             float d = 0.0f;
 #pragma unroll
-            for (int i = 0; i < L::frags; ++i) {
-                if constexpr (sizeof(T) == 2) {
-                    const uint32_t x[4] = {of[i].x, of[i].y, of[i].z, of[i].w}, y[4] = {df[r][i].x, df[r][i].y, df[r][i].z, df[r][i].w};
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        d = fmaf(__uint_as_float(x[e] << 16), __uint_as_float(y[e] << 16), d);
-                        d = fmaf(__uint_as_float(x[e] & 0xffff0000u), __uint_as_float(y[e] & 0xffff0000u), d);
-                    }
-                } else {
-                    d = fmaf(of[i].x, df[r][i].x, d);
-                    d = fmaf(of[i].y, df[r][i].y, d);
-                    d = fmaf(of[i].z, df[r][i].z, d);
-                    d = fmaf(of[i].w, df[r][i].w, d);
-                }
-            }
+            for (int i = 0; i < L::frags; ++i) d = vec_dot(of[i], df[r][i], d);
             d += __shfl_xor(d, 16);
             d += __shfl_xor(d, 32);
             D[r] = d;
@@ -650,31 +729,51 @@ __global__ __launch_bounds__(256) void attn_general_dq(const Args<T> p) {
         if (part != 0) return;
         gather<HD, RT>(region, p.region, 0, p.split, acc);
     }
+    unsigned redo = 0;  // as the forward's
+    T* out = p.out0 + (tok0 + q0 + c) * p.ld0 + hoff + 4 * g;
 #pragma unroll
     for (int r = 0; r < RT; ++r) {
-        const unsigned redo = non_finite<HD, RT>(acc, r);
-        for (int u = 0; u < 16; ++u) {
-            const int qi = q0 + 16 * r + u;
-            if (!((redo >> u) & 1) || qi >= p.Sq) continue;
-            const Row<T, HD> qr(p.q + (tok0 + qi) * p.ldq + hoff), dr(p.dout + (tok0 + qi) * p.ldo + hoff);
-            const float D = dr.dot(Row<T, HD>(p.o + (tok0 + qi) * p.ldo + hoff));
-            const float lse = p.lse[(static_cast<int64_t>(b) * p.H + h) * p.Sq + qi];
-            float da = 0.0f, db = 0.0f;
-            for (int key = 0; key < min(p.Sk, qi + p.coff + 1); ++key) {
-                const Row<T, HD> kr(kh + key * p.ldk);
-                const float ds = exp_of<T>(fmaf(qr.dot(kr), p.scale, -lse)) * (dr.dot(Row<T, HD>(vh + key * p.ldk)) - D);
-                da = fmaf(ds, kr.a, da);
-                db = fmaf(ds, kr.b, db);
-            }
-            store_row<T, HD>(p.out0 + (tok0 + qi) * p.ld0 + hoff, da * p.scale, db * p.scale);
-        }
-        const int qi = q0 + 16 * r + c;
-        if (qi >= p.Sq || ((redo >> c) & 1)) continue;
-        T* out = p.out0 + (tok0 + qi) * p.ld0 + hoff;
+        const unsigned bad = non_finite<HD, RT>(acc, r) & numbers(lse[r]) & numbers(D[r]);
+        redo |= bad << (16 * r);
+        if (q0 + 16 * r + c >= p.Sq || ((bad >> c) & 1)) continue;
 #pragma unroll
         for (int dt = 0; dt < HD / 16; ++dt) {
             const f32x4 a = acc[dt][r] * p.scale;
-            store4<VEC>(out + 16 * dt + 4 * g, a[0], a[1], a[2], a[3]);
+            store4<VEC>(out + 16 * r * p.ld0 + 16 * dt, a[0], a[1], a[2], a[3]);
+        }
+    }
+#pragma unroll 1
+    for (int r = 0; r < RT; ++r) {
+        if (!((redo >> (16 * r)) & 0xffffu)) continue;
+        const int qi = q0 + 16 * r + c, end = min(p.Sk, qi + p.coff + 1);
+        const int kend = min(p.Sk, min(q0 + 16 * r + 16, p.Sq) + p.coff);
+        const float lr = RT > 1 && r ? lse[RT - 1] : lse[0], Dr = RT > 1 && r ? D[RT - 1] : D[0];
+        typename L::Vec qf[L::frags], df[L::frags], f[L::frags];
+        load_row<T, HD, VEC>(p.q + tok0 * p.ldq + hoff, min(qi, p.Sq - 1), p.ldq, qf);
+        load_row<T, HD, VEC>(p.dout + tok0 * p.ldo + hoff, min(qi, p.Sq - 1), p.ldo, df);
+        f32x4 sum[HD / 16] = {};
+        for (int k0 = 0; k0 < kend; k0 += kRows) {
+            float x[2][4];
+            wait_lds();
+#pragma unroll
+            for (int t = 0; t < 2; ++t) {
+                const int row = min(k0 + 16 * t + c, p.Sk - 1);
+                load_row<T, HD, VEC>(vh, row, p.ldk, f);
+                const f32x4 dp = dot<HD>(f, df);
+                load_row<T, HD, VEC>(kh, row, p.ldk, f);
+                store_lds<T, HD>(region, 16 * t + c, f);
+                const f32x4 s = dot<HD>(f, qf);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) x[t][i] = exp_of<T>(fmaf(s[i], p.scale, -lr)) * (dp[i] - Dr);
+            }
+            wait_lds();
+            outer<T, HD>(region, x, [&](int row) { return k0 + row < end; }, sum);
+        }
+        if (qi >= p.Sq || !((redo >> (16 * r + c)) & 1)) continue;
+#pragma unroll
+        for (int dt = 0; dt < HD / 16; ++dt) {
+            const f32x4 a = sum[dt] * p.scale;
+            store4<VEC>(out + 16 * r * p.ld0 + 16 * dt, a[0], a[1], a[2], a[3]);
         }
     }
 }
@@ -765,34 +864,77 @@ __global__ __launch_bounds__(256) void attn_general_dkdv(const Args<T> p) {
         gather<HD, RT>(region, p.region, 0, p.split, dk);
         gather<HD, RT>(region, p.region, ACC, p.split, dv);
     }
+    unsigned redo = 0;  // as the forward's
+    const int64_t row0 = static_cast<int64_t>(b) * p.kb + k0 + c;
+    T *out_k = p.out0 + row0 * p.ld0 + hoff + 4 * g, *out_v = p.out1 + row0 * p.ld1 + hoff + 4 * g;
+    int nan_lse = -2, nan_D = -2;  // the last query whose lse, D is NaN; -2: not looked for yet
 #pragma unroll
     for (int r = 0; r < RT; ++r) {
-        const unsigned redo = non_finite<HD, RT>(dk, r) | non_finite<HD, RT>(dv, r);
-        for (int u = 0; u < 16; ++u) {
-            const int key = k0 + 16 * r + u;
-            if (!((redo >> u) & 1) || key >= p.Sk) continue;
-            const int64_t row = static_cast<int64_t>(b) * p.kb + key;
-            const Row<T, HD> kr(p.k + row * p.ldk + hoff), vr(p.v + row * p.ldk + hoff);
-            float ka = 0.0f, kb = 0.0f, va = 0.0f, vb = 0.0f;
-            for (int qi = max(0, key - p.coff); qi < p.Sq; ++qi) {
-                const Row<T, HD> qr(qh + qi * p.ldq), dr(dh + qi * p.ldo);
-                const float w = exp_of<T>(fmaf(qr.dot(kr), p.scale, -lse_h[qi])), ds = w * (dr.dot(vr) - D_h[qi]);
-                va = fmaf(w, dr.a, va);
-                vb = fmaf(w, dr.b, vb);
-                ka = fmaf(ds, qr.a, ka);
-                kb = fmaf(ds, qr.b, kb);
+        const unsigned bad_k = non_finite<HD, RT>(dk, r), bad_v = non_finite<HD, RT>(dv, r);
+        if ((bad_k | bad_v) && nan_lse == -2) {
+            nan_lse = nan_D = -1;
+#pragma unroll 4
+            for (int qi = lane; qi < p.Sq; qi += 64) {
+                if (lse_h[qi] != lse_h[qi]) nan_lse = qi;
+                if (D_h[qi] != D_h[qi]) nan_D = qi;
             }
-            store_row<T, HD>(p.out0 + row * p.ld0 + hoff, ka * p.scale, kb * p.scale);
-            store_row<T, HD>(p.out1 + row * p.ld1 + hoff, va, vb);
+#pragma unroll
+            for (int o = 1; o < 64; o *= 2) {
+                nan_lse = max(nan_lse, __shfl_xor(nan_lse, o));
+                nan_D = max(nan_D, __shfl_xor(nan_D, o));
+            }
         }
-        const int key = k0 + 16 * r + c;
-        if (key >= p.Sk || ((redo >> c) & 1)) continue;
-        const int64_t row = static_cast<int64_t>(b) * p.kb + key;
+        // a NaN lse that the key is seen with makes both sums NaN, a NaN D dK's
+        const int key = k0 + 16 * r + c, first = max(0, key - p.coff);
+        const bool bad = nan_lse < first && ((((nan_D < first ? bad_k : 0u) | bad_v) >> c) & 1);
+        redo |= static_cast<unsigned>(__ballot(bad) & 0xffffu) << (16 * r);
+        if (key >= p.Sk || bad) continue;
 #pragma unroll
         for (int dt = 0; dt < HD / 16; ++dt) {
             const f32x4 a = dk[dt][r] * p.scale, d = dv[dt][r];
-            store4<VEC>(p.out0 + row * p.ld0 + hoff + 16 * dt + 4 * g, a[0], a[1], a[2], a[3]);
-            store4<VEC>(p.out1 + row * p.ld1 + hoff + 16 * dt + 4 * g, d[0], d[1], d[2], d[3]);
+            store4<VEC>(out_k + 16 * r * p.ld0 + 16 * dt, a[0], a[1], a[2], a[3]);
+            store4<VEC>(out_v + 16 * r * p.ld1 + 16 * dt, d[0], d[1], d[2], d[3]);
+        }
+    }
+#pragma unroll 1
+    for (int r = 0; r < RT; ++r) {
+        if (!((redo >> (16 * r)) & 0xffffu)) continue;
+        const int key = k0 + 16 * r + c;
+        const int64_t krow = min(key, p.Sk - 1);
+        typename L::Vec kf[L::frags], vf[L::frags], f[L::frags];
+        load_row<T, HD, VEC>(p.k + static_cast<int64_t>(b) * p.kb * p.ldk + hoff, krow, p.ldk, kf);
+        load_row<T, HD, VEC>(p.v + static_cast<int64_t>(b) * p.kb * p.ldk + hoff, krow, p.ldk, vf);
+        f32x4 sk[HD / 16] = {}, sv[HD / 16] = {};
+        for (int q0 = max(0, k0 + 16 * r - p.coff) / kRows * kRows; q0 < p.Sq; q0 += kRows) {
+            float x[2][4], y[2][4];
+            wait_lds();
+#pragma unroll
+            for (int t = 0; t < 2; ++t) {
+                const int row = min(q0 + 16 * t + c, p.Sq - 1);
+                load_row<T, HD, VEC>(qh, row, p.ldq, f);
+                store_lds<T, HD>(region, 16 * t + c, f);
+                const f32x4 s = dot<HD>(f, kf);
+                load_row<T, HD, VEC>(dh, row, p.ldo, f);
+                store_lds<T, HD>(region_d, 16 * t + c, f);
+                const f32x4 dp = dot<HD>(f, vf);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const int qi = min(q0 + 16 * t + 4 * g + i, p.Sq - 1);
+                    x[t][i] = exp_of<T>(fmaf(s[i], p.scale, -lse_h[qi]));
+                    y[t][i] = x[t][i] * (dp[i] - D_h[qi]);
+                }
+            }
+            wait_lds();
+            auto seen = [&](int row) { return q0 + row < p.Sq && key <= q0 + row + p.coff; };
+            outer<T, HD>(region_d, x, seen, sv);
+            outer<T, HD>(region, y, seen, sk);
+        }
+        if (key >= p.Sk || !((redo >> (16 * r + c)) & 1)) continue;
+#pragma unroll
+        for (int dt = 0; dt < HD / 16; ++dt) {
+            const f32x4 a = sk[dt] * p.scale, d = sv[dt];
+            store4<VEC>(out_k + 16 * r * p.ld0 + 16 * dt, a[0], a[1], a[2], a[3]);
+            store4<VEC>(out_v + 16 * r * p.ld1 + 16 * dt, d[0], d[1], d[2], d[3]);
         }
     }
 }

@@ -104,3 +104,60 @@ def test_attention_infinities_stay_where_they_are_seen(dt):
     for got in (dirty, worse):
         for a, b in zip(got, clean):
             assert rel(a[:S - 1], b[:S - 1]) < tol
+
+
+def _visible_only(q, k, v, do, scale):
+    """Causal attention and its gradients in float64, each sum over exactly the rows that are seen."""
+    S, D = q.shape
+    o, dq, dk, dv = (np.zeros((S, D)) for _ in range(4))
+    lse = np.zeros(S)
+    P, dS = np.zeros((S, S)), np.zeros((S, S))
+    for i in range(S):
+        s = k[:i + 1] @ q[i] * scale
+        m = np.fmax.reduce(s)
+        lse[i] = m + np.log(np.sum(np.exp(s - m)))
+        P[i, :i + 1] = np.exp(s - lse[i])
+        o[i] = np.sum(P[i, :i + 1, None] * v[:i + 1], 0)
+    for i in range(S):
+        dS[i, :i + 1] = P[i, :i + 1] * (v[:i + 1] @ do[i] - do[i] @ o[i])
+        dq[i] = np.sum(dS[i, :i + 1, None] * k[:i + 1], 0) * scale
+    for j in range(S):
+        dk[j] = np.sum(dS[j:, j, None] * q[j:], 0) * scale
+        dv[j] = np.sum(P[j:, j, None] * do[j:], 0)
+    return dict(o=o, dq=dq, dk=dk, dv=dv)
+
+
+INF, NAN = float("inf"), float("nan")
+POISON = {"value": [("v", 36, 5, INF)], "first output gradient": [("do", 0, 5, INF)], "first query": [("q", 0, slice(None), NAN)],
+          "first rows": [("q", 0, slice(None), NAN), ("do", 0, slice(None), NAN)], "key": [("k", 20, 3, INF)],
+          "two values": [("v", 3, 7, -INF), ("v", 3, 9, NAN)], "all": [(n, slice(None), slice(None), NAN) for n in "q k v do".split()]}
+
+
+@pytest.mark.parametrize("dt", [F32, BF16])
+@pytest.mark.parametrize("D", [16, 32, 64, 128])
+@pytest.mark.parametrize("poison", POISON)
+def test_non_finite_rows_as_in_float64(dt, D, poison):
+    """Every output and gradient of 70 causal tokens with infinities or NaN in some rows: the same
+    entries infinite and NaN as in float64 over the visible rows alone, and the rest within the bounds
+    of finite inputs (rows next to a non-finite one are formed row by row, in fp32)."""
+    t, S = torch.float32 if dt == F32 else torch.bfloat16, 70
+    g = torch.Generator(device="cuda").manual_seed(D)
+    x = {n: torch.randn((S, D), generator=g, device="cuda").to(t) for n in ("q", "k", "v", "do")}
+    for n, r, c, val in POISON[poison]:
+        x[n][r, c] = val
+    o, lse = torch.empty_like(x["q"]), torch.empty((1, 1, S), device="cuda")
+    dq, dk, dv = (torch.empty_like(o) for _ in range(3))
+    scale = 1.0 / np.sqrt(D)
+    shape = (1, 1, S, S, D, 1, scale, dt, stream())
+    q, k, v, do = (x[n].data_ptr() for n in ("q", "k", "v", "do"))
+    call("aic_hip_attn_fwd_qk", q, D, k, v, D, o.data_ptr(), D, lse.data_ptr(), *shape)
+    call("aic_hip_attn_bwd_qk", q, D, k, v, D, o.data_ptr(), do, D, lse.data_ptr(), dq.data_ptr(), D, dk.data_ptr(), dv.data_ptr(), D,
+         *shape)
+    with np.errstate(all="ignore"):
+        want = _visible_only(*(host(x[n]).astype(np.float64) for n in ("q", "k", "v", "do")), scale)
+    for n, got in dict(o=host(o), dq=host(dq), dk=host(dk), dv=host(dv)).items():
+        ref = want[n]
+        assert np.array_equal(np.isfinite(got), np.isfinite(ref)) and np.array_equal(np.isnan(got), np.isnan(ref)), n
+        assert np.array_equal(got[np.isinf(got)], ref[np.isinf(ref)]), n
+        ok = np.isfinite(ref)
+        assert rel(got[ok], ref[ok]) < (2e-5 if dt == F32 else 8e-3), n
