@@ -413,9 +413,11 @@ void gemm_q4(const GemmArgs& a, hipStream_t s) {
 }
 
 // Rows that the fused RoPE / SwiGLU epilogues take: whole 256-row tiles, or any where the product
-// runs the persistent kernel (launch_dma), whose ragged form ends inside a tile.
+// runs the persistent kernel (launch_dma, which checks), whose ragged form ends inside a tile: RoPE and
+// SwiGLU on x W^T, SwiGLU's backward on dy W.
 bool rows_fuse(const GemmArgs& a) {
-    return a.M % 256 == 0 || (!a.Bq && a.r2 == 0 && !a.transA && a.K % 128 == 0 && a.K >= 256);
+    return a.M % 256 == 0 || (!a.Bq && a.r2 == 0 && !a.transA && (a.transB != 0) == !a.dglu_gu && a.K % 128 == 0 &&
+                              a.K >= 256);
 }
 
 void run_f32(const GemmArgs& a, hipStream_t s) {
