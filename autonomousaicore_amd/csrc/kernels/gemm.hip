@@ -8,8 +8,8 @@
 // This file holds the dispatch (tile shape, split-K, grouped and expert-ragged launches), the
 // split-K reduction and the SIMT kernel; the bf16 MFMA kernels are in gemm_kernels.inc,
 // instantiated per operand layout and output type by gemm_{nt,nn,tn,tt}_{bf16,f32}.hip.
-// fp32 operands run gemm_f32.hip, up to 64 rows of x W^T gemm_skinny.hip; bf16 operands whose layout
-// the matrix kernels do not take, a plain SIMT tiled kernel.
+// fp32 products run gemm_f32.hip, most of up to 64 rows of x W^T gemm_skinny.hip; fp32 operands with bf16
+// output and bf16 operands whose layout the matrix kernels do not take, a plain SIMT tiled kernel.
 #include "gemm.hpp"
 
 #include <algorithm>
@@ -445,15 +445,16 @@ bool try_skinny(const GemmArgs& a, hipStream_t s) {
         // A block's eight waves walk all of K, 1 ns a column and 0.045 more for each row, so a long K is
         // better cut among tile blocks, by more than the tiles' own fill and an epilogue's pass (64
         // rows: 16 columns over K 5632 25 us here, 11 there; 16 over 32768 147 and 21; eight rows: 2048 over
-        // 5632 9.9 and 11.7, 256 over 8192 13.2 and 13.1, 64 over 16384 24.4 and 15.6).  Past 2^25 weights
-        // the tile copies read W faster (16 rows of 32000x2048: 26.9 us here, 21.1 there); not where
-        // their epilogue would round the bf16 product before it adds R or C.
+        // 5632 9.9 and 11.7, 256 over 8192 13.2 and 13.1, 64 over 16384 24.4 and 15.6).
         const bool fused = a.rope_cos || a.glu_f > 0;
-        const int64_t t128 = (a.N + 127) / 128;
-        const int parts = stream_scratch_ready(s) ? dma_splits(t128, a) : 1;
-        if (a.K * (1e-3 + 4.5e-5 * a.M) > dma_us(a, parts) + (fused ? 6.5 : 2.5)) return false;
+        const double us = a.K * (1e-3 + 4.5e-5 * a.M) - (fused ? 6.5 : 2.5);
+        if (us > 4.0 && stream_scratch_ready(s) && us > dma_us(a, dma_splits((a.N + 127) / 128, a))) return false;
+        // Past 2^25 weights the tile copies read W faster (32000x2048: eight rows 27.1 us here and 20.9
+        // there, 16 rows 27.7 and 21.1); not where their epilogue would round the bf16 product before it
+        // adds R or C, and for fewer rows not by enough to keep other streams off the CUs (four
+        // rows 26.9 and 20.9, a decoding step 283 and 279 us, with three models at a time 308 and 310).
         const bool adds = a.c == DType::BFloat16 && (a.R || a.beta != 0.0f);
-        if (!fused && !adds && a.N * a.K > (int64_t{1} << 25)) return false;
+        if (!fused && !adds && a.M >= 8 && a.N * a.K > (int64_t{1} << 25)) return false;
     }
     SkinnyArgs q;
     q.g = a;
@@ -491,8 +492,8 @@ void gemm(const GemmArgs& a, hipStream_t s) {
     if (a.sq_part) {
         AIC_CHECK(a.c == DType::Float32 && a.sq_nf && a.sq_cap > 0 && !a.rope_cos && a.glu_f == 0 && !a.dglu_gu,
                   InvalidArgument, "GEMM sums of squares: fp32 output only, without the RoPE / SwiGLU epilogues");
-        // in the DMA tile kernels' epilogue or split-K reduction; the other paths (INT4 B, a
-        // low-rank term, the non-DMA kernels) read the product back
+        // in the epilogue of the DMA tile kernels and of gemm_f32, or in the reduction of K parts; the
+        // other paths (INT4 B, a low-rank term, the non-DMA kernels) read the product back
         if (gemm_f32_has_sq(a)) {
             run_f32(a, s);
             return;
