@@ -11,6 +11,7 @@ torch = pytest.importorskip("torch")
 pytestmark = pytest.mark.gpu
 
 import autonomousaicore_amd as aic  # noqa: E402
+from tests import torch_ref  # noqa: E402
 from tests.gpu_util import rel  # noqa: E402
 from tests.test_gpu_step import TINY, build, build_moe, build_qlora, make_base, make_lora, make_params, oracle_cfg  # noqa: E402
 
@@ -71,6 +72,45 @@ def test_moe_and_qlora_decode():
     steps = np.concatenate([q.forward_step(ids[:, p:p + 1], p) for p in range(20)], axis=1)
     assert rel(steps, full) < 1e-4
     q.close()
+
+
+def _with_adapters(cfg, dense, lora, r, alpha):
+    """The dense model whose projections are W + alpha / r B A."""
+    out, pos, off = dense.astype(np.float64), {}, 0
+    for name, shape in torch_ref.layout(cfg["vocab"], cfg["d"], cfg["L"], cfg["f"], cfg["tied"]):
+        pos[name] = (off, shape)
+        off += int(np.prod(shape))
+    ad, off = {}, 0
+    for name, shape in torch_ref.lora_layout(cfg["d"], cfg["L"], cfg["f"], r):
+        ad[name] = lora[off:off + int(np.prod(shape))].reshape(shape).astype(np.float64)
+        off += int(np.prod(shape))
+    for name in ad:
+        if name.endswith("lora_A"):
+            pre = name[:-len("lora_A")]
+            at, shape = pos[pre + "weight"]
+            out[at:at + int(np.prod(shape))] += (alpha / r * ad[pre + "lora_B"] @ ad[name]).reshape(-1)
+    return out.astype(np.float32)
+
+
+@pytest.mark.parametrize("d,H,f,L,B", [(640, 5, 704, 2, 1), (640, 5, 704, 2, 4), (2048, 16, 768, 1, 16)])
+def test_bf16_qlora_decode(orc, d, H, f, L, B):
+    """INT4 base and adapters in bf16: a chunk, single tokens, a chunk and a token against the oracle's
+    forward over the whole sequence, at widths of one to four norm chunks a row (640 and 704 end inside one;
+    16 rows of 2048 are the largest normalised block).  The bound is the dense bf16 test's."""
+    cfg, S, r, alpha, G = dict(vocab=512, d=d, L=L, H=H, f=f, tied=False), 14, 16, 32.0, 128
+    m = build_qlora(cfg, r, alpha, G, compute="bfloat16")
+    base, lora = make_base(m, 61, std=0.04), make_lora(m, 67, 0.02)
+    m.set_base_params(base)
+    m.set_params(lora)
+    ids, _ = aic.batch(13, B, S, cfg["vocab"])
+    ocfg = oracle_cfg(orc, cfg, S)
+    dense = _with_adapters(cfg, orc.qlora_dequantize_base(ocfg, G, base), lora, r, alpha)
+    ref = orc.lm_logits(ocfg, dense, ids, B, S)
+    cuts = [0, 5, 6, 7, 8, 9, 12, 13, S]
+    got = np.concatenate([m.forward_step(ids[:, a:b], a) for a, b in zip(cuts, cuts[1:])], axis=1)
+    for t in range(S):
+        assert rel(got[:, t], ref[:, t]) < 3e-2, t
+    m.close()
 
 
 def test_generate_greedy_follows_the_oracle_argmax(orc):
