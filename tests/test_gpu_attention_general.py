@@ -66,7 +66,7 @@ def test_attention_tile_edges(orc, dt, B, H, Sq, Sk, D, causal, pad, shift):
     for name, got, ref in zip("q k v".split(), (heads(dq, Sq), heads(dk, Sk), heads(dv, Sk)),
                               orc.flash_bwd(Q, K, V, O, DO, L, causal)):
         # one key: dS = P (dP - D) cancels exactly in the reference; then the bound is absolute
-        assert rel(got, ref) < tol or np.max(np.abs(got - ref)) < tol, name
+        assert np.max(np.abs(got - ref)) < tol if Sk == 1 else rel(got, ref) < tol, name
     for buf, x in ((bo, o), (bdq, dq), (bdk, dk), (bdv, dv)):  # nothing outside the heads was written
         inside = np.zeros(buf.numel(), bool)
         inside[shift:shift + x.numel()].reshape(x.shape)[:, :H * D] = True

@@ -1,8 +1,8 @@
-"""The general attention forward with the keys of a few queries shared by several blocks: from 25
-blocks of 32 keys up (800 keys leave one partial, 801 take the first key of the next), with uneven
-shares, a causal offset, an infinity that one block sees, and inside a graph capture on a stream
-without scratch memory, where one block keeps all keys.  Bounds as for the same entry at its tile
-edges: fp32 sums, and one bf16 rounding of the outputs."""
+"""The general attention forward with the keys of a few queries shared by several blocks: where a
+head's row times the blocks of 32 keys passes 2816 bytes, so past 704 keys of 128 bytes (bf16 heads of
+64) and 352 of 256 (bf16 heads of 128, fp32 heads of 64), with uneven shares, a causal offset, an
+infinity that one block sees, and inside a graph capture, where one block keeps all keys.  Bounds as for
+the same entry at its tile edges: fp32 sums, and one bf16 rounding of the outputs."""
 import numpy as np
 import pytest
 
@@ -43,7 +43,10 @@ def _heads(x, B, S, H, D):
 @pytest.mark.parametrize("dt", [F32, BF16])
 @pytest.mark.parametrize("B,H,Sq,Sk,D,causal", [(1, 2, 1, 768, 64, False), (1, 2, 1, 769, 64, False),
                                                 (2, 3, 1, 801, 128, False), (1, 2, 16, 1100, 32, True),
-                                                (1, 1, 7, 4100, 16, True), (8, 16, 1, 1500, 64, False)])
+                                                (1, 1, 7, 4100, 16, True), (8, 16, 1, 1500, 64, False),
+                                                (1, 2, 1, 704, 64, False), (1, 2, 1, 705, 64, False),
+                                                (1, 2, 3, 352, 128, False), (1, 2, 3, 353, 128, False),
+                                                (1, 2, 1, 352, 64, False), (1, 2, 1, 353, 64, False)])
 def test_attention_key_parts(orc, dt, B, H, Sq, Sk, D, causal):
     q, k, v = _ops(B, H, Sq, Sk, D, dt)
     o, lse = _fwd(q, k, v, B, H, Sq, Sk, D, causal, dt)
