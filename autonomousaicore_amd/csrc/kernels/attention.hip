@@ -968,9 +968,11 @@ void attn_bwd_qk(const void* q, int64_t ld_q, const void* k, const void* v, int6
 void attn_cached(const void* q, int64_t ldq, const void* kc, const void* vc, int64_t ldkv, int64_t cache_rows, void* o,
                  int64_t ldo, int64_t B, int64_t H, int64_t S_new, int64_t start_pos, int64_t hd, float scale, DType dt,
                  hipStream_t s) {
-    AIC_CHECK(B >= 0 && H > 0 && S_new >= 0 && start_pos >= 0 && hd > 0 && hd <= 128 && 256 % hd == 0 &&
+    AIC_CHECK(B >= 0 && H > 0 && S_new >= 0 && start_pos >= 0 && (hd == 16 || hd == 32 || hd == 64 || hd == 128) &&
                   ldq >= H * hd && ldkv >= H * hd && ldo >= H * hd,
               InvalidArgument, "attn_cached: bad shape");
+    // 16384 positions: what this entry has always taken (its first kernel kept a row's scores in LDS; the
+    // one behind it now has no such limit)
     AIC_CHECK(start_pos + S_new <= cache_rows && start_pos + S_new <= 16384, InvalidArgument,
               "attn_cached: the cache holds ", cache_rows, " positions (at most 16384), needed ", start_pos + S_new);
     if (B == 0 || S_new == 0) return;

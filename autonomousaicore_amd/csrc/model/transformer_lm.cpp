@@ -1098,7 +1098,7 @@ void TransformerLM::forward_backward(const int64_t* ids, const int64_t* targets,
     };
     auto slots = [&](int64_t r) { return SqSlots{sq_part_ + r * sq_region_, sq_nf_ + r * sq_region_, sq_region_}; };
     // every slot starts at zero: a launch writes only the slots of its path, which can change with
-    // the token count (T not a multiple of 64 leaves the tile kernels)
+    // the token count (tile shape, K parts)
     if (fold) {
         auto _p = prof_.scope(kGradNorm, 0.0, 12.0 * sq_slots_, s);
         hip::sqnorm_clear(sq_part_, sq_nf_, sq_slots_, s);
