@@ -53,6 +53,38 @@ __device__ __forceinline__ void sq_add1(double& acc, int& nf, float v) {
     nf |= (__float_as_uint(v) & 0x7f800000u) == 0x7f800000u;
 }
 
+// V partials of consecutive elements, summed over the K parts in part order.
+template <int V>
+struct alignas(4 * V) Partials {
+    float v[V];
+    __device__ __forceinline__ void add(const Partials& p) {
+#pragma unroll
+        for (int e = 0; e < V; ++e) v[e] += p.v[e];
+    }
+};
+template <int V>
+__device__ __forceinline__ Partials<V> sum_parts(const float* P, int splits, int64_t pz) {
+    auto part = [&](int z) { return *reinterpret_cast<const Partials<V>*>(P + z * pz); };
+    Partials<V> acc = part(0);
+    int z = 1;
+    // eight loads in flight, added in z order
+    for (; z + 8 <= splits; z += 8) {
+        Partials<V> p[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) p[u] = part(z + u);
+#pragma unroll
+        for (int u = 0; u < 8; ++u) acc.add(p[u]);
+    }
+    Partials<V> rest[7];
+#pragma unroll
+    for (int u = 0; u < 7; ++u)
+        if (z + u < splits) rest[u] = part(z + u);
+#pragma unroll
+    for (int u = 0; u < 7; ++u)
+        if (z + u < splits) acc.add(rest[u]);
+    return acc;
+}
+
 // C = alpha * sum_z P[z] + beta * C + R over the split-K partials P [splits][M][N] (fp32,
 // summed in z order: deterministic); with sq, each block also writes the sum of squares of
 // the values it stored (one slot per block).  V elements of a row per thread: 4 (16-byte loads) where
@@ -63,47 +95,21 @@ __device__ __forceinline__ void sq_add1(double& acc, int& nf, float v) {
 // order; 256x2304 14.0 (17.1 with 4-byte loads in row order), 1000x768 in four of 512 14.6 (17.4).
 template <typename CT, int V>
 __global__ __launch_bounds__(256) void splitk_reduce_k(const float* __restrict__ P, int splits, int64_t pz, int M, int N,
-                                                       int tile, int wshift, int tiles_m, int tiles_n, float alpha,
-                                                       float beta, CT* C, int64_t ldc, const CT* R, int64_t ldr,
-                                                       double* sq, int* sq_nf) {
-    struct alignas(4 * V) FV {
-        float v[V];
-    };
+                                                       int tile, int tiles_m, int tiles_n, float alpha, float beta,
+                                                       CT* C, int64_t ldc, const CT* R, int64_t ldr, double* sq,
+                                                       int* sq_nf) {
     struct alignas(sizeof(CT) * V) CV {
         CT v[V];
     };
-    int tm = xcd_id(blockIdx.x, gridDim.x), tn = 0;
-    if (tiles_n > 1) tile_of(blockIdx.x, gridDim.x, tiles_m, tiles_n, tm, tn);
-    // stripes of 1 << wshift columns (divisions by a variable take 0.1 us each at this kernel's start)
-    const int rows = 256 * V >> wshift, at = static_cast<int>(threadIdx.x) * V;
-    const int n = tn * tile + (at & ((1 << wshift) - 1)), end = n < N ? min((tm + 1) * tile, M) : 0;
+    int tm, tn;
+    tile_of(blockIdx.x, gridDim.x, tiles_m, tiles_n, tm, tn);
+    const int rows = 256 * V / tile, n = tn * tile + static_cast<int>(threadIdx.x) * V % tile;
+    const int end = n < N ? min((tm + 1) * tile, M) : 0;
     double sqa = 0.0;
     int sqf = 0;
-    for (int m = tm * tile + static_cast<int>(blockIdx.y) * rows + (at >> wshift); m < end;
+    for (int m = tm * tile + static_cast<int>(blockIdx.y) * rows + static_cast<int>(threadIdx.x) * V / tile; m < end;
          m += rows * static_cast<int>(gridDim.y)) {
-        const int64_t i = static_cast<int64_t>(m) * N + n;
-        auto partial = [&](int z) { return *reinterpret_cast<const FV*>(P + z * pz + i); };
-        FV acc = partial(0);
-        auto add = [&](const FV& p) {
-#pragma unroll
-            for (int e = 0; e < V; ++e) acc.v[e] += p.v[e];
-        };
-        int z = 1;
-        // eight loads in flight, added in z order
-        for (; z + 8 <= splits; z += 8) {
-            FV p[8];
-#pragma unroll
-            for (int u = 0; u < 8; ++u) p[u] = partial(z + u);
-#pragma unroll
-            for (int u = 0; u < 8; ++u) add(p[u]);
-        }
-        FV rest[7];
-#pragma unroll
-        for (int u = 0; u < 7; ++u)
-            if (z + u < splits) rest[u] = partial(z + u);
-#pragma unroll
-        for (int u = 0; u < 7; ++u)
-            if (z + u < splits) add(rest[u]);
+        const Partials<V> acc = sum_parts<V>(P + static_cast<int64_t>(m) * N + n, splits, pz);
         CT* c = C + static_cast<int64_t>(m) * ldc + n;
         CV old{}, res{}, out;
         if (beta != 0.0f) old = *reinterpret_cast<const CV*>(c);
@@ -122,6 +128,31 @@ __global__ __launch_bounds__(256) void splitk_reduce_k(const float* __restrict__
         const unsigned slot = blockIdx.y * gridDim.x + blockIdx.x;
         sq_block256(sqa, sqf, sq + slot, sq_nf + slot);
     }
+}
+
+// The same for at most kFewResults elements, one per thread in row order: finding the tile costs more than
+// their sums, and a tile's stripes leave most lanes of narrow rows idle.  Product and reduction, in tile
+// order and here: 65x16 over K 5632 12.1 and 11.0 us, 128x16 over 2048 11.4 and 10.5, 65x768 over 2048
+// 10.8 and 10.1, 8192x16 over 1536 12.8 and 11.9, 1024x64 over 2048 14.6 and 14.3; from 131072 elements up
+// the order of the tiles pays.
+constexpr int64_t kFewResults = 131072;
+template <typename CT>
+__global__ __launch_bounds__(256) void splitk_reduce_few_k(const float* __restrict__ P, int splits, int M, int N,
+                                                           float alpha, float beta, CT* C, int64_t ldc, const CT* R,
+                                                           int64_t ldr, double* sq, int* sq_nf) {
+    const int i = static_cast<int>(blockIdx.x * 256 + threadIdx.x);
+    double sqa = 0.0;
+    int sqf = 0;
+    if (i < M * N) {
+        const int m = i / N, n = i % N;
+        const int64_t at = static_cast<int64_t>(m) * ldc + n;
+        float v = alpha * sum_parts<1>(P + i, splits, static_cast<int64_t>(M) * N).v[0];
+        if (beta != 0.0f) v += beta * ld(C, at);
+        if (R) v += ld(R, static_cast<int64_t>(m) * ldr + n);
+        st(C, at, v);
+        if (sq) sq_add1(sqa, sqf, v);
+    }
+    if (sq) sq_block256(sqa, sqf, sq + blockIdx.x, sq_nf + blockIdx.x);
 }
 
 // Sums of squares of the fp32 matrix C [M, N] (leading dimension ldc), one slot per block: the
@@ -275,45 +306,47 @@ void splitk_reduce(const float* part, int splits, int tile, const GemmArgs& a, h
     const bool vec = a.N % 4 == 0 && a.ldc % 4 == 0 && reinterpret_cast<uintptr_t>(a.C) % (4 * es) == 0 &&
                      (!a.R || (a.ldr % 4 == 0 && reinterpret_cast<uintptr_t>(a.R) % (4 * es) == 0)) &&
                      reinterpret_cast<uintptr_t>(part) % 16 == 0;
-    const int64_t tm = (a.M + tile - 1) / tile, tn = (a.N + tile - 1) / tile, tiles = tm * tn;
-    int wshift = 2;  // columns of a stripe: the tile's, or where N ends early the power of two that holds them
-    while (1 << wshift < tile && int64_t{1} << wshift < a.N) ++wshift;
-    const int64_t stripes = std::max<int64_t>(1, (int64_t{tile} << wshift) / (vec ? 1024 : 256));
-    const int64_t gy = std::max<int64_t>(1, std::min<int64_t>(stripes, (a.sq_part ? 1024 : 4096) / tiles));
-    const int64_t grid = tiles * gy;
-    AIC_CHECK(grid < (int64_t{1} << 31), InvalidArgument, "split-K reduction: too many tiles");
-    auto launch = [&](auto tag, auto v) {
+    const bool few = total <= kFewResults, f32 = a.c == DType::Float32;
+    const int64_t tm = (a.M + tile - 1) / tile, tn = (a.N + tile - 1) / tile;
+    const int64_t gx = few ? (total + 255) / 256 : tm * tn, stripes = int64_t{tile} * tile / (vec ? 1024 : 256);
+    const int64_t gy = few ? 1 : std::max<int64_t>(1, std::min<int64_t>(stripes, (a.sq_part ? 1024 : 4096) / gx));
+    AIC_CHECK(gx * gy < (int64_t{1} << 31), InvalidArgument, "split-K reduction: too many tiles");
+    AIC_CHECK(!f32 || !a.sq_part || (a.sq_nf && gx * gy <= a.sq_cap), InvalidArgument, "GEMM sums of squares: ", gx * gy,
+              " slots needed, ", a.sq_cap, " given");
+    const dim3 grid(static_cast<unsigned>(gx), static_cast<unsigned>(gy));
+    const int M = static_cast<int>(a.M), N = static_cast<int>(a.N);
+    auto launch = [&](auto tag) {
         using CT = decltype(tag);
-        hipLaunchKernelGGL((splitk_reduce_k<CT, decltype(v)::value>),
-                           dim3(static_cast<unsigned>(tiles), static_cast<unsigned>(gy)), dim3(256), 0, s, part, splits,
-                           total, static_cast<int>(a.M), static_cast<int>(a.N), tile, wshift, static_cast<int>(tm),
-                           static_cast<int>(tn), a.alpha, a.beta, static_cast<CT*>(a.C), a.ldc,
-                           static_cast<const CT*>(a.R), a.ldr, a.c == DType::Float32 ? a.sq_part : nullptr,
-                           a.c == DType::Float32 ? a.sq_nf : nullptr);
+        CT* C = static_cast<CT*>(a.C);
+        const CT* R = static_cast<const CT*>(a.R);
+        double* sq = f32 ? a.sq_part : nullptr;
+        int* nf = f32 ? a.sq_nf : nullptr;
+        if (few) {
+            hipLaunchKernelGGL(splitk_reduce_few_k<CT>, grid, dim3(256), 0, s, part, splits, M, N, a.alpha, a.beta, C, a.ldc,
+                               R, a.ldr, sq, nf);
+            return;
+        }
+        void (*kernel)(const float*, int, int64_t, int, int, int, int, int, float, float, CT*, int64_t, const CT*, int64_t,
+                       double*, int*) = vec ? splitk_reduce_k<CT, 4> : splitk_reduce_k<CT, 1>;
+        hipLaunchKernelGGL(kernel, grid, dim3(256), 0, s, part, splits, total, M, N, tile, static_cast<int>(tm),
+                           static_cast<int>(tn), a.alpha, a.beta, C, a.ldc, R, a.ldr, sq, nf);
     };
-    auto by_width = [&](auto tag) {
-        if (vec) launch(tag, std::integral_constant<int, 4>{});
-        else launch(tag, std::integral_constant<int, 1>{});
-    };
-    if (a.c == DType::Float32) {
-        AIC_CHECK(!a.sq_part || (a.sq_nf && grid <= a.sq_cap), InvalidArgument, "GEMM sums of squares: ", grid,
-                  " slots needed, ", a.sq_cap, " given");
-        by_width(float{});
-    } else {
-        by_width(bf16{});
-    }
+    if (f32) launch(float{});
+    else launch(bf16{});
     AIC_LAUNCH_CHECK("splitk_reduce_k");
 }
 
 // K parts of a product on 128x128 tiles of which one block fits a CU: few tiles over a long K fill
 // the chip with parts of it (the partials summed in a fixed order afterwards), at most one round of
 // blocks.  The part count with the least of: the chain along K, 6 ns a step of one column (measured
-// from K 768 to 8192), and, with parts, the reduction's launch and fill (4 us) and its traffic
-// (0.35 us per MB of partials).  2304x768 over K 1024 in one part 12.1 us (two parts, which any
-// product of fewer than 128 tiles was cut into, 18.4); 768x768 over K 8192 in four parts 22.6 (eight,
-// more than a round, 30.8; one 53.7); 1000x768 over K 3072 in four 16.4 (one 23.0).
+// from K 768 to 8192), and, with parts, the reduction's launch and fill (4 us, 2.8 for few results)
+// and its traffic (0.35 us per MB of partials).  2304x768 over K 1024 in one part 12.1 us (two parts,
+// which any product of fewer than 128 tiles was cut into, 18.4); 65x8 over 1024 in two 9.9 (one 10.4);
+// 768x768 over K 8192 in four parts 22.6 (eight, more than a round, 30.8; one 53.7); 1000x768 over
+// K 3072 in four 16.4 (one 23.0).
 double dma_us(const GemmArgs& a, int parts) {
-    return 6e-3 * a.K / parts + (parts > 1 ? 4.0 + 1.4e-6 * parts * a.M * a.N : 0.0);
+    const int64_t total = a.M * a.N;
+    return 6e-3 * a.K / parts + (parts > 1 ? (total <= kFewResults ? 2.8 : 4.0) + 1.4e-6 * parts * total : 0.0);
 }
 int dma_splits(int64_t t128, const GemmArgs& a) {
     int best = 1;
@@ -448,7 +481,7 @@ bool try_skinny(const GemmArgs& a, hipStream_t s) {
         // 5632 9.9 and 11.7, 256 over 8192 13.2 and 13.1, 64 over 16384 24.4 and 15.6).
         const bool fused = a.rope_cos || a.glu_f > 0;
         const double us = a.K * (1e-3 + 4.5e-5 * a.M) - (fused ? 6.5 : 2.5);
-        if (us > 4.0 && stream_scratch_ready(s) && us > dma_us(a, dma_splits((a.N + 127) / 128, a))) return false;
+        if (us > 2.8 && stream_scratch_ready(s) && us > dma_us(a, dma_splits((a.N + 127) / 128, a))) return false;
         // Past 2^25 weights the tile copies read W faster (32000x2048: eight rows 27.1 us here and 20.9
         // there, 16 rows 27.7 and 21.1); not where their epilogue would round the bf16 product before it
         // adds R or C, and for fewer rows not by enough to keep other streams off the CUs (four

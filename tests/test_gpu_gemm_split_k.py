@@ -1,7 +1,7 @@
 """Dense products whose K is cut into parts, around the limits of the reduction: tiles that end
-inside a stripe, rows whose width or leading dimension rules out four-element loads, beta and a
-residual, each output type, and inside a graph capture on a stream without scratch memory (one
-part).  The operands are small integers, so the float32 sums are exact in any order."""
+inside a stripe, rows whose width or leading dimension rules out four-element loads, 131072 results
+and fewer (reduced in row order) and more, beta and a residual, each output type, and inside a graph
+capture on a stream without scratch memory (one part).  The operands are small integers, so the float32 sums are exact in any order."""
 import pytest
 
 torch = pytest.importorskip("torch")
@@ -43,7 +43,8 @@ def _run(M, N, K, pad, ct, beta, residual, ta=0, st=None, capture=None):
 @pytest.mark.parametrize("ct", [F32, BF16])
 @pytest.mark.parametrize("M,N,K,pad,beta,residual", [(128, 512, 4096, 0, 0.0, False), (129, 516, 4096, 4, 1.0, True),
                                                      (70, 130, 8192, 1, 0.0, True), (1000, 768, 2560, 0, 1.0, False),
-                                                     (1000, 2304, 4096, 8, 0.0, True)])
+                                                     (1000, 2304, 4096, 8, 0.0, True), (256, 512, 4096, 0, 1.0, True),
+                                                     (257, 512, 4096, 0, 1.0, True), (40, 24, 16384, 1, 1.0, True)])
 def test_split_k_reduction(ct, M, N, K, pad, beta, residual):
     _run(M, N, K, pad, ct, beta, residual)
 
