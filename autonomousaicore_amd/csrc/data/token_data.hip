@@ -193,6 +193,7 @@ int64_t TokenLoader::next_device(int64_t* inputs, int64_t* targets, hipStream_t 
     if (st.in_flight) AIC_HIP_CHECK(hipEventSynchronize(st.copied));  // its previous copy has finished
     if (resident_) {
         for (int64_t i = 0; i < b; ++i) st.host[i] = ds_->window_start(samples[static_cast<size_t>(i)]);
+        const StreamScratchUse use(s);
         int64_t* starts = static_cast<int64_t*>(stream_scratch(sizeof(int64_t) * static_cast<size_t>(batch_), s, 6));
         AIC_HIP_CHECK(hipMemcpyAsync(starts, st.host, sizeof(int64_t) * static_cast<size_t>(b), hipMemcpyHostToDevice,
                                      s));

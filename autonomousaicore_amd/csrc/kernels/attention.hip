@@ -892,6 +892,7 @@ void attn_bwd(const void* q, const void* k, const void* v, int64_t ld_qkv, const
     if (B == 0 || S == 0) return;
     if (dt == DType::BFloat16 && mfma_ok(q, k, v, ld_qkv, dout, ld_o, hd) && ld_d % 8 == 0 && a16(dq) && a16(dk) &&
         a16(dv) && a16(o)) {
+        const StreamScratchUse use(s);
         float* D = static_cast<float*>(stream_scratch(sizeof(float) * B * H * S, s));
         // the dQ kernel computes D = rowsum(dO * O) for its queries and writes it for dK/dV
         const float sl2 = scale * kLog2e;

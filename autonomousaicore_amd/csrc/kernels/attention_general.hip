@@ -993,6 +993,7 @@ void launch(Args<T> p, hipStream_t s) {
     p.region = p.split > 1 ? REGION : ALONE;
     int64_t grid = (per + waves / p.split - 1) / (waves / p.split) * nbh;
     p.parts = 1;
+    const StreamScratchUse use(s);
     if (K == kFwd && RT == 1 && per == 1 && p.split == max_waves) {
         p.parts = key_parts(nbh, (std::min<int64_t>(p.Sk, p.Sq + static_cast<int64_t>(p.coff)) + kRows - 1) / kRows,
                             static_cast<int64_t>(sizeof(T)) * HD);
@@ -1073,6 +1074,7 @@ void bwd(const GenAttn& a, hipStream_t s) {
     p.o = static_cast<const T*>(a.o);
     p.dout = static_cast<const T*>(a.dout);
     p.lse = const_cast<float*>(a.lse);
+    const StreamScratchUse use(s);
     // no queries: the key kernel's empty loop writes zero dK and dV
     p.D = static_cast<float*>(stream_scratch(sizeof(float) * std::max<int64_t>(a.B * a.H * a.Sq, 1), s));
     p.ldq = a.ldq; p.ldk = a.ldk; p.ldo = a.ldo;

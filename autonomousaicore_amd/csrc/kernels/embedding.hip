@@ -458,6 +458,7 @@ void embed_bwd(const int64_t* ids, int64_t N, const void* dout, int64_t V, int64
     for (int b : {16, 8, 4})
         if (!lb && row_bytes % (64 * b) == 0 && (reinterpret_cast<uintptr_t>(dout) % b) == 0) lb = b;
     const bool runs = lb > 0 && vec;
+    const StreamScratchUse use(s);
     int* spos = static_cast<int*>(stream_scratch(sizeof(int) * (4 * N + 3), s));
     int* sid = spos + N;
     int* rstart = sid + N;      // N + 1 entries

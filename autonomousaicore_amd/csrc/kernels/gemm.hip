@@ -426,6 +426,7 @@ void gemm_q4(const GemmArgs& a, hipStream_t s) {
         splits = 2;  // two of these blocks fit a CU
     }
     if (splits > 1 && stream_scratch_ready(s)) {
+        const StreamScratchUse use(s);
         float* part = static_cast<float*>(stream_scratch(partial_bytes(a, splits), s, 7));
         a.transB ? gemm_impl::launch_dma_q4<128, 128, 64, 2, true, float>(a, s, splits, part)
                  : gemm_impl::launch_dma_q4<128, 128, 64, 2, false, float>(a, s, splits, part);
@@ -459,6 +460,7 @@ void run_f32(const GemmArgs& a, hipStream_t s) {
         gemm_f32(a, s);
         return;
     }
+    const StreamScratchUse use(s);
     float* partial = static_cast<float*>(stream_scratch(partial_bytes(a, parts), s, 7));
     gemm_f32(a, s, parts, partial);
     splitk_reduce(partial, parts, 64, a, s);
@@ -557,6 +559,7 @@ void gemm(const GemmArgs& a, hipStream_t s) {
                                           : (a.rope_hd == 128 || a.rope_hd == 64) && gemm_impl::kDmaWaves256 == 8 &&
                                                 gemm_dma_eligible(a) && a.r2 == 0);
         if (!fused) {
+            const StreamScratchUse use(s);  // w, until the product is launched
             GemmArgs b = a;
             b.rope_cos = b.rope_sin = nullptr;
             if (a.Bq && !gemm_q4_eligible(a)) {
@@ -654,6 +657,7 @@ void gemm(const GemmArgs& a, hipStream_t s) {
             }
         }
         if (splits256 > 1 && stream_scratch_ready(s)) {
+            const StreamScratchUse use(s);
             float* part = static_cast<float*>(stream_scratch(partial_bytes(a, splits256), s, 7));
             dispatch_dma<256, 256, 64, 2, float>(a, s, splits256, part);
             splitk_reduce(part, splits256, 256, a, s);
@@ -661,6 +665,7 @@ void gemm(const GemmArgs& a, hipStream_t s) {
         }
         const int splits = plain && !big ? dma_splits(t128, a) : 1;
         if (splits > 1 && stream_scratch_ready(s)) {
+            const StreamScratchUse use(s);
             float* part = static_cast<float*>(stream_scratch(partial_bytes(a, splits), s, 7));
             dispatch_dma<128, 128, 64, 4, float>(a, s, splits, part);
             splitk_reduce(part, splits, 128, a, s);

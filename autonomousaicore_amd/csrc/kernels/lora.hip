@@ -460,6 +460,7 @@ void lora_skinny(const LoraSkinny& q, hipStream_t s) {
     }
     const int64_t groups = chunks / p.cpb, row_blocks = (q.T + p.tt - 1) / p.tt;
     const int64_t gps = cps / p.cpb, segs = q.N / q.n_seg;
+    const StreamScratchUse use(s);
     if (p1 && gps > 1) p.p1 = static_cast<float*>(stream_scratch(sizeof(float) * groups * q.T * q.r_seg, s, 2));
     if (p2 && row_blocks > 1)
         p.p2 = static_cast<float*>(stream_scratch(sizeof(float) * row_blocks * q.N * q.r_seg, s, 3));

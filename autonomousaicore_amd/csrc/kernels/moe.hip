@@ -562,6 +562,7 @@ void moe_route(const float* logits, int64_t T, int64_t E, int64_t k, float aux_c
     AIC_LAUNCH_CHECK("moe_route");
     // statistics: kStatsTokens tokens per block, then the partials in block order
     const int nparts = static_cast<int>((T + kStatsTokens - 1) / kStatsTokens);
+    const StreamScratchUse use(s);
     double* part_p = static_cast<double*>(stream_scratch((sizeof(double) + sizeof(long long)) * nparts * E, s));
     long long* part_c = reinterpret_cast<long long*>(part_p + static_cast<int64_t>(nparts) * E);
     hipLaunchKernelGGL(moe_stats_k, dim3(static_cast<unsigned>(nparts)), dim3(kStatsTokens), 0, s, idx, probs,

@@ -419,6 +419,7 @@ void bwd_t(const void* dy, int64_t lddy, const void* x, int64_t ldx, const float
     const int ch = chunks_for(dim, VN);
     const int rpw = static_cast<int>(bwd_rows_per_wave(rows));
     const unsigned grid = static_cast<unsigned>(rmsnorm_bwd_part_rows(rows));
+    const StreamScratchUse use(s);
     float* part = ext_part;  // the caller's partial rows (reduced later), or scratch reduced below
     if (dw && !part) part = static_cast<float*>(stream_scratch(sizeof(float) * grid * dim, s));
     const size_t lds = dw ? sizeof(float) * 4 * dim : 0;

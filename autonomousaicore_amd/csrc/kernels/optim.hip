@@ -346,6 +346,7 @@ void grad_sqnorm_multi(const float* const* grads, const int64_t* sizes, int coun
     AIC_CHECK(count <= kMaxNormTensors, InvalidArgument, "grad_sqnorm_multi: at most ", kMaxNormTensors, " tensors");
     int blocks[kMaxNormTensors];
     const int total = static_cast<int>(sqnorm_blocks(sizes, count, blocks));
+    const StreamScratchUse use(s);
     double* pd = static_cast<double*>(
         stream_scratch(sizeof(double) * std::max(total, 1) + sizeof(int) * std::max(total, 1), s));
     int* pn = reinterpret_cast<int*>(pd + std::max(total, 1));

@@ -82,7 +82,14 @@ std::map<std::tuple<int, hipStream_t, int>, ScratchEntry>& scratch_cache() {
 }
 }  // namespace
 
+StreamScratchUse::StreamScratchUse(hipStream_t stream) {
+    static std::recursive_mutex locks[64];
+    const auto h = reinterpret_cast<uintptr_t>(stream);
+    lock_ = std::unique_lock(locks[(h >> 4 ^ h >> 10) % 64]);
+}
+
 void stream_scratch_release(hipStream_t stream) {
+    const StreamScratchUse use(stream);
     std::lock_guard<std::mutex> lk(scratch_mu);
     auto& cache = scratch_cache();
     for (auto it = cache.begin(); it != cache.end();) {

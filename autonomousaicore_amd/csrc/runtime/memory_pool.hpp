@@ -13,6 +13,7 @@
 
 #include <cstddef>
 #include <cstdint>
+#include <mutex>
 
 namespace aic {
 
@@ -65,9 +66,19 @@ private:
 // on one stream runs in order, so a kernel's scratch can be reused by the next call on the
 // same stream without a free and a new allocation (each of which costs a few microseconds of
 // stream time).  The pointer stays valid until the next call with the same key asks for more
-// bytes; callers use it only for the duration of their own launches.  Slots let one call hold
-// several buffers at once.
+// bytes; callers use it only for the duration of their own launches, under a StreamScratchUse.  Slots
+// let one call hold several buffers at once.
 void* stream_scratch(size_t bytes, hipStream_t stream, int slot = 0);
+// Held from before stream_scratch to the last launch that uses the buffer: a call of another thread on
+// the same stream would otherwise write it between this call's launches, or hand it back to the pool
+// before them.  Recursive; streams share a fixed set of locks.
+class StreamScratchUse {
+public:
+    explicit StreamScratchUse(hipStream_t stream);
+
+private:
+    std::unique_lock<std::recursive_mutex> lock_;
+};
 // Whether work on `stream` may use stream_scratch where another form does without: not while the
 // stream is captured.  A graph would keep the buffer's address, and the buffer goes back to the pool
 // when a later call needs a larger one or the stream's buffers are released.
