@@ -29,10 +29,10 @@
 // MFMA pipe and LDS reads with 13 products where 7 are counted (the split probabilities).  Forward
 // and backward of 64 heads of 128, 128 queries on 2048 keys, bf16: 172 us (32.1 ms with the
 // one-thread-per-row kernels before); 512 queries 0.52 ms (74.8), fp32 1.83 ms (48.3); one query of
-// 12 heads of 64 on 2048 keys 10 us (6.1 ms).  Error against 64 bits, beside the
-// fp32 probabilities and expf of those kernels, over 40 shapes in bf16 (1 to 512 queries, 16 to 2048
-// keys): o and dv 1.7e-3 in both to four digits, dq and dk within 0.2% either way, lse 7e-8 and at the
-// median 0.87 of theirs; fp32 1.0e-6 (1.2e-6).
+// 12 heads of 64 on 2048 keys 10 us (6.1 ms).  Error against 64 bits, beside the fp32 probabilities
+// and expf of those kernels, over 40 shapes in bf16 (1 to 512 queries, 16 to 2048 keys): o and dv
+// 1.7e-3 in both to four digits, dq and dk within 0.2% either way, lse 7e-8 and at the median 0.87 of
+// theirs; fp32 1.0e-6 (1.2e-6).
 #include <algorithm>
 #include <cmath>
 #include <type_traits>

@@ -98,7 +98,7 @@ void gemm(const GemmArgs& a, hipStream_t stream);
 // (norm_w, [K]: op(A) = A / rms(A) * w, at most 16 rows); the k and v columns of a q/k/v product
 // also stored to the KV cache (kc, vc: [batch][kv_rows][d]; row m is position rope_start + m %
 // rope_seq of sequence m / rope_seq); skip_c: only glu_out is written.  gemm() runs them on this
-// path by itself where it can.
+// path by itself where it can and the tile kernels are not faster.
 constexpr int64_t kSkinnyRows = 64;
 struct SkinnyArgs {
     GemmArgs g;
